@@ -47,7 +47,6 @@ int ensure_xstage(size_t bytes, const char* op);   // P0_OK, or an error (no roo
 // per-file set-up at p0_open (kernel attributes; the no-allocation GEMM's scratch address)
 int gemm_init();
 int gemv_init();
-int misc_init();
 
 // Thread-local message of the last failure (p0_last_error).
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));

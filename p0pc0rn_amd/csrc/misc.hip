@@ -1,7 +1,13 @@
 // misc.hip - the GEMV's producer and consumers in a decode step: row statistics (the rstd slot an rms prologue reads),
 // the split-K sum with the residual RMS update (normadd), and the argmax over the per-tile maxima a softcap GEMV
-// writes. One workgroup of 256 threads per row, summing in the reference's order (thread t takes elements t, t + 256,
-// ... in turn, then a halving tree over the 256 partials), so the fp32 sums equal the reference's, bit for bit.
+// writes. rowstats and normadd sum in the reference's order (256 partials, partial t over elements t, t + 256, ... in
+// turn, then a halving tree), so the fp32 sums equal the reference's, bit for bit.
+//
+// One wave owns a row: lane l holds the partials 4 l .. 4 l + 3, so 256 consecutive elements are one 16-byte load per
+// lane, and the whole tree is lane moves within the wave (no LDS, no barrier). Bound: at a decode step's one row, the
+// memory round trips (launch, loads, stores); at thousands of rows, HBM bandwidth. A workgroup of 256 threads per row
+// with one 4-byte load in flight per thread and nine barriers a tree took, per launch, 11.5 us for a normadd of 2048
+// values over 1 or 4 partials and 24.7 us for the statistics of 4608 x 3072 values; this takes 4.1 and 11.7 (4.9 TB/s).
 #include "common.hpp"
 
 // no FMA contraction: every a + b * c rounds the product and the sum separately, as the CPU restatement does, so the
@@ -10,119 +16,269 @@
 
 namespace p0 {
 
-constexpr int kRowThreads = 256;
+constexpr int kChunk = 256;   // elements a wave takes per step: 4 consecutive ones per lane
 
-// the reference's halving tree over red[0..255] (engine/ops/misc.js:20-23, engine/llm/lops.js:158-159): level s adds
-// red[t + s] into red[t] for t < s; every thread gets red[0]
-__device__ __forceinline__ float tree256(float v, float* red) {
-  const int t = threadIdx.x;
-  red[t] = v;
-  __syncthreads();
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+// the reference's halving tree over 256 partials (engine/ops/misc.js:20-23, engine/llm/lops.js:158-159: level s adds
+// red[t + s] to red[t]), partial 4 l + c in component c of lane l; every lane gets the result. Levels 128 and 64 pair
+// lanes 32 and 16 apart, 32 .. 4 lanes 8 .. 1 apart (a rotation by s of a row whose values have period 2 s is the
+// exchange with lane ^ s), 2 and 1 the components.
+__device__ __forceinline__ float tree256(const float (&part)[4]) {
+  float v[4];
 #pragma unroll
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s) red[t] = red[t] + red[t + s];
-    __syncthreads();
+  for (int c = 0; c < 4; ++c) {
+    float t = part[c];
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+    t = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(t), __float_as_uint(t), false, false);
+    t = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    t = t + dpp_move<0x128>(t);   // row_ror:8
+    t = t + dpp_move<0x124>(t);
+    t = t + dpp_move<0x122>(t);
+    v[c] = t + dpp_move<0x121>(t);
   }
-  const float r = red[0];
-  __syncthreads();
-  return r;
+  return (v[0] + v[2]) + (v[1] + v[3]);
 }
 
 __device__ __forceinline__ float rsqrt_exact(float v) { return 1.0f / __builtin_sqrtf(v); }
 
+// elements i .. i + 3 of the n at a (0 past their end). VEC: 16-byte aligned rows of a multiple of 4 elements
+template <bool VEC>
+__device__ __forceinline__ float4 load4(const float* __restrict__ a, int i, int n) {
+  if (VEC) return i < n ? *(const float4*)(a + i) : float4{0.0f, 0.0f, 0.0f, 0.0f};
+  float4 v;
+  v.x = i < n ? a[i] : 0.0f;
+  v.y = i + 1 < n ? a[i + 1] : 0.0f;
+  v.z = i + 2 < n ? a[i + 2] : 0.0f;
+  v.w = i + 3 < n ? a[i + 3] : 0.0f;
+  return v;
+}
+__device__ __forceinline__ float at(const float4& v, int c) { return c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w; }
+
+// NB chunks of a row are held in registers (ONCE: a row of at most NB 256 elements, read once); longer rows run in
+// batches of NB chunks and are read again in the second pass. An element past the row's end adds 0 to a sum that is
+// never -0, which leaves its bits alone; terms that are not plain elements are left out instead.
 // engine/ops/misc.js:17-30
-__global__ __launch_bounds__(kRowThreads) void rowstats_kernel(const float* __restrict__ x, int64_t ld, int64_t c0,
-                                                              int64_t rows, int64_t cols, int mode, float eps,
-                                                              float* __restrict__ st, int64_t st_off) {
-  __shared__ float red[kRowThreads];
-  const int t = threadIdx.x;
-  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+template <bool VEC, int NB, bool ONCE>
+__global__ __launch_bounds__(256) void rowstats_kernel(const float* __restrict__ x, int64_t ld, int64_t c0,
+                                                       int64_t rows, int64_t cols, int mode, float eps,
+                                                       float* __restrict__ st, int64_t st_off) {
+  const int lane = threadIdx.x & 63;
+  const int64_t step = (int64_t)gridDim.x * (blockDim.x >> 6);
+  for (int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); row < rows; row += step) {
     const float* xr = x + row * ld + c0;
-    float mean = 0.0f;
-    if (mode == 0) {
-      float s = 0.0f;
-      for (int64_t i = t; i < cols; i += kRowThreads) s = s + xr[i];
-      mean = tree256(s, red) / (float)cols;
+    float4 v[NB];
+    auto load = [&](int64_t b) -> int {   // the batch at b; its length
+      const int n = (int)(cols - b < NB * kChunk ? cols - b : NB * kChunk);
+#pragma unroll
+      for (int k = 0; k < NB; ++k) v[k] = load4<VEC>(xr + b, k * kChunk + 4 * lane, n);
+      return n;
+    };
+    float q[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mean = 0.0f;
+    auto sums = [&](float (&s)[4]) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) s[c] = s[c] + at(v[k], c);
+    };
+    auto squares = [&](int n) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float d = at(v[k], c) - mean;
+          q[c] = k * kChunk + 4 * lane + (VEC ? 0 : c) < n ? q[c] + d * d : q[c];
+        }
+    };
+    if (ONCE) {
+      const int n = load(0);
+      if (mode == 0) {
+        float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        sums(s);
+        mean = tree256(s) / (float)cols;
+      }
+      squares(n);
+    } else {
+      if (mode == 0) {
+        float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int64_t b = 0; b < cols; b += NB * kChunk) {
+          load(b);
+          sums(s);
+        }
+        mean = tree256(s) / (float)cols;
+      }
+      for (int64_t b = 0; b < cols; b += NB * kChunk) squares(load(b));
     }
-    float q = 0.0f;
-    for (int64_t i = t; i < cols; i += kRowThreads) {
-      const float d = xr[i] - mean;
-      q = q + d * d;
-    }
-    const float var = tree256(q, red) / (float)cols;
-    if (t == 0) {
+    const float var = tree256(q) / (float)cols;
+    if (lane == 0) {
       st[(st_off + row) * 2] = mean;
       st[(st_off + row) * 2 + 1] = rsqrt_exact(var + eps);
     }
   }
 }
 
-// engine/llm/lops.js:153-170; the t sums of a row live in LDS (dynamic: D floats)
-__global__ __launch_bounds__(kRowThreads) void normadd_kernel(const float* __restrict__ T, int64_t nsrc, int64_t ldp,
-                                                             const float* __restrict__ W, int64_t woff,
-                                                             float* __restrict__ X, float* __restrict__ ST,
-                                                             int64_t stoff, int64_t D, float eps, float scale,
-                                                             int mode) {
-  __shared__ float red[kRowThreads];
-  extern __shared__ float tv[];
-  const int t = threadIdx.x;
+// engine/llm/lops.js:153-170. ONCE: the row's partials (four at a time), its residual and the norm weights are all in
+// flight together before the first sum; longer rows add the partials again in the second pass (the same order, the
+// same bits).
+template <bool VEC, int NB, bool ONCE>
+__global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T, int64_t nsrc, int64_t ldp,
+                                                     const float* __restrict__ W, int64_t woff, float* X,
+                                                     float* __restrict__ ST, int64_t stoff, int64_t D, float eps,
+                                                     float scale, int mode) {
+  const int lane = threadIdx.x;
   const int64_t m = blockIdx.x, xb = m * D;
-  float s = 0.0f;
-  for (int64_t i = t; i < D; i += kRowThreads) {
-    float v = 0.0f;
-    for (int64_t j = 0; j < nsrc; ++j) v = v + T[j * ldp + xb + i];
-    tv[i] = v;
-    s = s + v * v;
+  float4 t[NB], xv[NB], wv[NB];
+  auto length = [&](int64_t b) { return (int)(D - b < NB * kChunk ? D - b : NB * kChunk); };
+  auto tsum = [&](int64_t b) {   // the partials in j order
+    const int n = length(b);
+#pragma unroll
+    for (int k = 0; k < NB; ++k) t[k] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto add = [&](const float4 (&v)[NB]) {
+#pragma unroll
+      for (int k = 0; k < NB; ++k) {
+        t[k].x = t[k].x + v[k].x;
+        t[k].y = t[k].y + v[k].y;
+        t[k].z = t[k].z + v[k].z;
+        t[k].w = t[k].w + v[k].w;
+      }
+    };
+    int64_t j = 0;
+    for (; j + 4 <= nsrc; j += 4) {
+      float4 v[4][NB];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int k = 0; k < NB; ++k) v[u][k] = load4<VEC>(T + (j + u) * ldp + xb + b, k * kChunk + 4 * lane, n);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(v[u]);
+    }
+    for (; j < nsrc; ++j) {
+      float4 v[NB];
+#pragma unroll
+      for (int k = 0; k < NB; ++k) v[k] = load4<VEC>(T + j * ldp + xb + b, k * kChunk + 4 * lane, n);
+      add(v);
+    }
+  };
+  auto inputs = [&](int64_t b) {
+    const int n = length(b);
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      xv[k] = wv[k] = float4{0.0f, 0.0f, 0.0f, 0.0f};
+      if (mode == 0) {
+        xv[k] = load4<VEC>(X + xb + b, k * kChunk + 4 * lane, n);
+        wv[k] = load4<VEC>(W + woff + b, k * kChunk + 4 * lane, n);
+      }
+    }
+  };
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f}, s2[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto squares = [&] {
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[c] = s[c] + at(t[k], c) * at(t[k], c);
+  };
+  if (ONCE) {
+    inputs(0);
+    tsum(0);
+    squares();
+  } else {
+    for (int64_t b = 0; b < D; b += NB * kChunk) {
+      tsum(b);
+      squares();
+    }
   }
-  const float rs = rsqrt_exact(tree256(s, red) / (float)D + eps);
-  float s2 = 0.0f;
-  for (int64_t i = t; i < D; i += kRowThreads) {
-    float xv = X[xb + i];
-    if (mode == 0) xv = (xv + tv[i] * rs * W[woff + i]) * scale;
-    else xv = tv[i];
-    X[xb + i] = xv;
-    s2 = s2 + xv * xv;
+  const float rs = rsqrt_exact(tree256(s) / (float)D + eps);
+  auto update = [&](int64_t b) {
+    const int n = length(b);
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int i = k * kChunk + 4 * lane;
+      float y[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        y[c] = mode == 0 ? (at(xv[k], c) + at(t[k], c) * rs * at(wv[k], c)) * scale : at(t[k], c);
+        s2[c] = i + (VEC ? 0 : c) < n ? s2[c] + y[c] * y[c] : s2[c];
+      }
+      if (VEC) {
+        if (i < n) *(float4*)(X + xb + b + i) = float4{y[0], y[1], y[2], y[3]};
+      } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (i + c < n) X[xb + b + i + c] = y[c];
+      }
+    }
+  };
+  if (ONCE) {
+    update(0);
+  } else {
+    for (int64_t b = 0; b < D; b += NB * kChunk) {
+      inputs(b);
+      tsum(b);
+      update(b);
+    }
   }
-  const float r2 = tree256(s2, red);
-  if (t == 0) ST[stoff + m] = rsqrt_exact(r2 / (float)D + eps);
+  const float r2 = tree256(s2);
+  if (lane == 0) ST[stoff + m] = rsqrt_exact(r2 / (float)D + eps);
 }
 
-// engine/llm/lops.js:418-433, engine/llm/lops_spec.js:329-343: (value, index) with ties to the lower index
+// engine/llm/lops.js:418-433, engine/llm/lops_spec.js:329-343: (value, index) with ties to the lower index. A running
+// best is never NaN, so "better" is a total order on what is combined: any order of the reduction gives its result. One
+// workgroup of 16 waves per row, four pairs in flight per thread (the 4096 tile maxima of a 262144-row head in one
+// round; 256 threads that loaded 16 pairs one after another took 6.3 us a launch, this 4.0).
+constexpr int kArgThreads = 1024;
+typedef uint32_t u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));   // an 8-byte load at 4-byte alignment
 __device__ __forceinline__ bool better(float v, uint32_t id, float bv, uint32_t bi) {
   return v > bv || (v == bv && id < bi);
 }
-__global__ __launch_bounds__(kRowThreads) void argmax_kernel(const float* __restrict__ MX, int64_t n,
+__device__ __forceinline__ void wave_best(float& v, uint32_t& id) {
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    const float ov = __shfl_xor(v, s, 64);
+    const uint32_t oi = (uint32_t)__shfl_xor((int)id, s, 64);
+    if (better(ov, oi, v, id)) { v = ov; id = oi; }
+  }
+}
+__global__ __launch_bounds__(kArgThreads) void argmax_kernel(const float* __restrict__ MX, int64_t n,
                                                             uint32_t* __restrict__ out) {
-  __shared__ float rv[kRowThreads];
-  __shared__ uint32_t ri[kRowThreads];
-  const int t = threadIdx.x;
-  const int64_t b = (int64_t)blockIdx.x * n;
+  __shared__ float rv[kArgThreads / 64];
+  __shared__ uint32_t ri[kArgThreads / 64];
+  const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
+  const float* row = MX + 2 * (int64_t)blockIdx.x * n;
   float bv = -3.4e38f;
   uint32_t bi = 0xFFFFFFFFu;
-  for (int64_t i = t; i < n; i += kRowThreads) {
-    const float v = MX[2 * (b + i)];
-    const uint32_t id = __float_as_uint(MX[2 * (b + i) + 1]);
-    if (better(v, id, bv, bi)) { bv = v; bi = id; }
+  for (int64_t i0 = 0; i0 < n; i0 += 4 * kArgThreads) {
+    u32x2a4 p[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int64_t i = i0 + u * kArgThreads + t;
+      p[u] = i < n ? *(const u32x2a4*)(row + 2 * i) : u32x2a4{0xFF800000u, 0xFFFFFFFFu};   // -inf: never better
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const float v = __uint_as_float(p[u].x);
+      if (better(v, p[u].y, bv, bi)) { bv = v; bi = p[u].y; }
+    }
   }
-  rv[t] = bv;
-  ri[t] = bi;
+  wave_best(bv, bi);
+  if (lane == 0) {
+    rv[wv] = bv;
+    ri[wv] = bi;
+  }
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (t < s && better(rv[t + s], ri[t + s], rv[t], ri[t])) { rv[t] = rv[t + s]; ri[t] = ri[t + s]; }
-    __syncthreads();
-  }
-  if (t == 0) {
-    out[2 * blockIdx.x] = ri[0];
-    out[2 * blockIdx.x + 1] = __float_as_uint(rv[0]);
+  if (wv != 0) return;
+  bv = rv[lane & (kArgThreads / 64 - 1)];
+  bi = ri[lane & (kArgThreads / 64 - 1)];
+  wave_best(bv, bi);
+  if (lane == 0) {
+    out[2 * blockIdx.x] = bi;
+    out[2 * blockIdx.x + 1] = __float_as_uint(bv);
   }
 }
 
-// normadd's LDS allowance (one row of up to 150 KB), set once at p0_open
-int misc_init() {
-  P0_HIP(hipFuncSetAttribute((const void*)normadd_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024),
-         "p0_open: normadd");
-  return P0_OK;
-}
+static bool vec_ok(const float* p, int64_t a, int64_t b) { return (((uintptr_t)p | (uintptr_t)(a * 4) | (uintptr_t)(b * 4)) & 15) == 0; }
 
 }  // namespace p0
 
@@ -140,10 +296,20 @@ extern "C" int p0_rowstats(const p0_rowstats_args_t* a) {
   if (building_chain())   // a chain op (chain_aux.hpp): the same sums in the same order
     return chain_add_rowstats((const float*)((const uint8_t*)a->x + a->x_off), ld, a->x_c0, a->rows, a->cols,
                               (int)a->mode, a->eps, a->st, a->st_off);
-  const unsigned grid = (unsigned)(a->rows < 65536 * 4 ? a->rows : 65536 * 4);
-  hipLaunchKernelGGL(rowstats_kernel, dim3(grid), dim3(kRowThreads), 0, ctx().cur,
-                     (const float*)((const uint8_t*)a->x + a->x_off), ld, a->x_c0, a->rows, a->cols, (int)a->mode,
-                     a->eps, a->st, a->st_off);
+  // one row per wave; four waves a workgroup once there are rows for more than the chip holds at one each (1024: the
+  // dispatch of thousands of one-wave workgroups is what shows then). 4096 columns stay in registers; a longer row is
+  // read again for its variance, 2048 columns at a time.
+  const float* x = (const float*)((const uint8_t*)a->x + a->x_off);
+  const int wpb = a->rows >= 1024 ? 4 : 1;
+  const int64_t blocks = (a->rows + wpb - 1) / wpb;
+  const unsigned grid = (unsigned)(blocks < 65536 * 4 ? blocks : 65536 * 4);
+  const bool vec = vec_ok(x, ld, a->x_c0) && a->cols % 4 == 0;
+  auto k = !vec                       ? rowstats_kernel<false, 4, false>
+           : a->cols <= 8 * kChunk    ? rowstats_kernel<true, 8, true>
+           : a->cols <= 16 * kChunk   ? rowstats_kernel<true, 16, true>
+                                      : rowstats_kernel<true, 8, false>;
+  hipLaunchKernelGGL(k, dim3(grid), dim3(64 * wpb), 0, ctx().cur, x, ld, a->x_c0, a->rows, a->cols, (int)a->mode, a->eps,
+                     a->st, a->st_off);
   P0_LAUNCHED("rowstats");
   return P0_OK;
 }
@@ -160,8 +326,9 @@ extern "C" int p0_normadd(const p0_normadd_args_t* a) {
   const float eps = a->eps != 0.0f ? a->eps : 1e-6f;
   if (building_chain())
     return chain_add_normadd(a->t, nsrc, ldp, a->w, a->w_off, a->x, a->st, a->st_off, D, M, eps, a->scale, (int)a->mode);
-  const size_t lds = (size_t)D * sizeof(float);
-  hipLaunchKernelGGL(normadd_kernel, dim3((unsigned)M), dim3(kRowThreads), lds, ctx().cur, a->t, nsrc, ldp, a->w,
+  const bool vec = vec_ok(a->t, ldp, D) && vec_ok(a->x, 0, 0) && (a->mode == 1 || vec_ok(a->w, a->w_off, 0));
+  auto k = !vec ? normadd_kernel<false, 4, false> : D <= 8 * kChunk ? normadd_kernel<true, 8, true> : normadd_kernel<true, 8, false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)M), dim3(64), 0, ctx().cur, a->t, nsrc, ldp, a->w,
                      a->w_off, a->x, a->st, a->st_off, D, eps, a->scale, (int)a->mode);
   P0_LAUNCHED("normadd");
   return P0_OK;
@@ -172,7 +339,7 @@ extern "C" int p0_argmaxM(const float* mx, int64_t n, int64_t M, uint32_t* out) 
   if (n < 0 || M < 1) { set_error("argmax: n %lld, M %lld", (long long)n, (long long)M); return P0_EINVAL; }
   if (int r = require_open("argmax")) return r;
   if (building_chain()) return chain_add_argmax(mx, n, M, out);
-  hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)M), dim3(kRowThreads), 0, ctx().cur, mx, n, out);
+  hipLaunchKernelGGL(argmax_kernel, dim3((unsigned)M), dim3(kArgThreads), 0, ctx().cur, mx, n, out);
   P0_LAUNCHED("argmax");
   return P0_OK;
 }

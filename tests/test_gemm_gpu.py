@@ -210,3 +210,33 @@ def test_gemm_flux_shape_sampled_rows(dev):
     check(y[rows].ravel(), ys, "FLUX QKV sampled rows", 1e-5)
     for b in (wb, xb, yb):
         b.free()
+
+
+@pytest.mark.parametrize("mode", ["f16", "bf16", "lnmod", "rms"])
+@pytest.mark.parametrize("M,K,pad", [(3, 544, 0), (9001, 32, 0), (33005, 32, 0), (2051, 2592, 1)])
+def test_gemm_staging_rows_per_wave(dev, mode, M, K, pad):
+    """the activation staging where a wave walks 1, 4 and 8 rows (3, 9001 and 33005 x one strip; 2051 x six, the last of
+    32 columns), with a ragged last row group, 16-byte aligned rows and rows that are not (a leading element). One fp32
+    rounding may differ from the oracle's before the value is rounded to fp16, which flips about 2^-12 of the fp16
+    roundings by 2^-11: 1.3e-5 relative; the bar is four times that"""
+    N, ld, c0 = 64, K + 8 * pad, pad if mode != "f16" else 1
+    ld += 1 if mode == "f16" else 0
+    w = _weights(N, K, 21)
+    xf = O.randn(M * ld, 10, 1.5)
+    x = (xf if mode in ("lnmod", "rms") else xf.astype(np.float16) if mode == "f16"
+         else (xf.view(np.uint32) >> 16).astype(np.uint16))
+    st = np.empty(2 * M, np.float32)
+    xr = xf.reshape(M, ld).astype(np.float64)
+    st[0::2] = xr.mean(1)
+    st[1::2] = 1 / np.sqrt(xr.var(1) + 1e-6)
+    pv = O.randn(2 * (K + 8), 16, 0.1)
+    f = dict(w_rows=N, w_cols=K, M=M, N=N, K=K, x_ld=ld, x_k0=c0, x_mode=capi.XMODE[mode], epi=capi.GEPI["f32"],
+             pv_off=K + 8, pv_stride=(1 << 32) - (K + 8))
+    f["x_ld"] = ld + (0 if c0 + K <= ld else 8)
+    if f["x_ld"] != ld:
+        x = np.concatenate([x.reshape(M, ld), np.zeros((M, 8), x.dtype)], 1).ravel()
+    arrays = dict(w=w, x=x)
+    if mode in ("lnmod", "rms"):
+        arrays.update(stats=st, pv=pv)
+    want, got = run(f, arrays, np.float32, M * N)
+    check(got, want, f"gemm staging {mode} {M}x{K}", 5e-5)

@@ -89,3 +89,42 @@ def test_argmax_of_a_softcap_gemv(dev):
     assert got[0] == int(np.argmax(logits)) and got[1] == logits.max().view(np.uint32)
     for b in (wb, xb, nb, mb, y, out):
         b.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (5, 252), (1027, 256), (3, 2048), (2, 2052), (5, 4096), (2, 4100), (1, 9000)])
+def test_rowstats_aligned_rows_bit_exact(dev, rows, cols, mode):
+    """16-byte aligned rows: a row held in registers (up to 2048 and 4096 columns), a longer one read twice, and the
+    four-rows-a-workgroup launch with a ragged last workgroup. The same order of sums as the oracle: equal bits"""
+    x = (2.0 + O.randn(rows * cols, 31 + cols)).astype(np.float32)
+    want = np.full(rows * 2, np.nan, np.float32)
+    O.rowstats(capi.rowstats_args(x=x.ctypes.data, rows=rows, cols=cols, mode=mode, eps=1e-5, st=want.ctypes.data))
+    xb = capi.to_device(x)
+    st = capi.Buffer(want.nbytes + 8).fill_u32(NAN)
+    capi.rowstats(capi.rowstats_args(x=xb, rows=rows, cols=cols, mode=mode, eps=1e-5, st=st))
+    got = st.read(np.float32).view(np.uint32)
+    assert np.array_equal(got[:2 * rows], want.view(np.uint32))
+    assert (got[2 * rows:2 * rows + 2] == NAN).all()
+    xb.free(); st.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("D,M,nsrc", [(4, 1, 1), (1000, 3, 5), (2048, 2, 8), (2052, 2, 4), (6148, 1, 3)])
+def test_normadd_aligned_rows_bit_exact(dev, D, M, nsrc, mode):
+    """16-byte aligned rows, in registers (up to 2048 values) and in two passes, partials in fours with a remainder"""
+    t = O.randn(nsrc * M * D, D + nsrc, 0.3).astype(np.float32)
+    w = (0.5 + O.rng_uniform(D, D)).astype(np.float32)
+    x0 = O.randn(M * D, D + 1).astype(np.float32)
+    xw, sw = x0.copy(), np.full(M, np.nan, np.float32)
+    kw = dict(t_n=nsrc, D=D, M=M, eps=1e-6, scale=0.9, mode=mode)
+    O.normadd(capi.normadd_args(t=t.ctypes.data, w=w.ctypes.data, x=xw.ctypes.data, st=sw.ctypes.data, **kw))
+    tb, wb, xb = capi.to_device(t), capi.to_device(w), capi.Buffer(x0.nbytes + 16).fill_u32(NAN)
+    xb.upload(x0)
+    sb = capi.Buffer(sw.nbytes).fill_u32(NAN)
+    capi.normadd(capi.normadd_args(t=tb, w=wb, x=xb, st=sb, **kw))
+    gx, gs = xb.read(np.float32).view(np.uint32), sb.read(np.float32, M).view(np.uint32)
+    assert np.array_equal(gx[:M * D], xw.view(np.uint32))
+    assert (gx[M * D:M * D + 4] == NAN).all()
+    assert np.array_equal(gs, sw.view(np.uint32))
+    for b in (tb, wb, xb, sb):
+        b.free()

@@ -111,3 +111,21 @@ def test_probe_read_reads_the_whole_buffer(dev):
         capi.probe_read(buf, n - 8, sink)
     buf.free()
     sink.free()
+
+
+@pytest.mark.parametrize("shift", [0, 1])
+@pytest.mark.parametrize("N,K", [(64, 32), (128, 256), (64, 288), (192, 1056)])
+def test_dequant_group_remainders_and_alignment(dev, N, K, shift):
+    """a last block of fewer than 8 groups, and outputs that are not 16-byte aligned; nothing past the outputs written"""
+    b, _ = O.pack_q4(O.randn(N * K, N + K, 0.05), N, K)
+    wb = capi.to_device(b)
+    o32, o16 = capi.Buffer(4 * N * K + 32).fill_u32(0x7FC00000), capi.Buffer(2 * N * K + 32).fill_u32(0x7FC07FC0)
+    capi.q4_dequant(wb, N, K, out32=o32.ptr + 4 * shift, out16=o16.ptr + 2 * shift)
+    g32, g16 = o32.read(np.uint32), o16.read(np.uint16)
+    w32, w16 = O.dequant_q4(b, N, K)
+    n = N * K
+    assert np.array_equal(g32[shift:n + shift], np.asarray(w32).ravel().view(np.uint32))
+    assert np.array_equal(g16[shift:n + shift], np.asarray(w16).ravel().view(np.uint16))
+    assert (g32[n + shift:n + 4] == 0x7FC00000).all() and (g16[n + 2:n + 8] == (0x7FC0)).all()
+    for x in (wb, o32, o16):
+        x.free()
