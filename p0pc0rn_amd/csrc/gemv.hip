@@ -5,6 +5,7 @@
 // the same arguments, the same split semantics (nsplit partial rows Y[split * ldy + m * ldm + n]) and the same errors.
 // The kernels and their mapping onto MI355X are described in gemv_kernels.hpp.
 #include "chain_aux.hpp"
+#include "gemvm.hpp"
 
 #include <algorithm>
 #include <map>
@@ -69,8 +70,7 @@ static Plan plan(int M, int NT, int epi, int nsplit, int kPer) {
   const int kws_max = Gs / g_min_gpw > 1 ? Gs / g_min_gpw : 1;
   if (kws > kws_max) kws = kws_max;
   if (kws < 1) kws = 1;
-  const bool mf = M >= 2 && M >= g_mf_min_m;   // the MFMA kernel (512 threads)
-  const int max_kw = M <= 2 && !mf ? g_max_kw : (g_max_kw < 8 ? g_max_kw : 8);   // the kernel's launch bound
+  const int max_kw = M <= 2 ? g_max_kw : (g_max_kw < 8 ? g_max_kw : 8);   // the kernel's launch bound
   pl.kw = kws < max_kw ? kws : max_kw;
   // one tile per slot whose K is split across workgroups anyway: at most 8 waves per slot, so that twice the
   // workgroups (each with half the records to issue and dot) share it
@@ -80,11 +80,9 @@ static Plan plan(int M, int NT, int epi, int nsplit, int kPer) {
   pl.waves = pl.tgw * pl.kw;
   int nks = (kws + pl.kw - 1) / pl.kw;
   int gps = (Gs + nks - 1) / nks;
-  // LDS: x' and its group sums for the slice, plus the reduction rows. M >= 2 runs on MFMA (gemv_item): its group
-  // sums take 16 entries per group (a 16-row A operand) when M < 16
+  // LDS: x' and its group sums for the slice, plus the reduction rows
   const size_t red = (size_t)pl.waves * T * 64 * sizeof(float);
-  const int XS = mf && M < 16 ? 16 : M;
-  int maxGps = (int)((48 * 1024 - red) / ((size_t)M * 32 * sizeof(float) + (size_t)XS * sizeof(float)));
+  int maxGps = (int)((48 * 1024 - red) / ((size_t)M * 33 * sizeof(float)));
   if (maxGps < 1) maxGps = 1;
   if (gps > maxGps) gps = maxGps;
   for (;;) {   // the partials must fit the workspace: coarser slices until they do
@@ -95,7 +93,7 @@ static Plan plan(int M, int NT, int epi, int nsplit, int kPer) {
   pl.gps = gps;
   pl.nks = nks;
   pl.ntb = (slots + pl.tgw - 1) / pl.tgw;
-  pl.lds = (size_t)M * gps * 32 * sizeof(float) + (size_t)XS * gps * sizeof(float) + red;
+  pl.lds = (size_t)M * gps * 33 * sizeof(float) + red;
   return pl;
 }
 
@@ -524,19 +522,11 @@ static bool plan_wide(std::vector<GemvP>& ops, int G) {
   return true;
 }
 
-// the q8 kernels' LDS allowance, set once at p0_open (never lazily, e.g. while the stream is being captured)
-int gemv_init() {
-  for (int M : {1, 2})
-    P0_HIP(hipFuncSetAttribute((const void*)q8_kernel(M), hipFuncAttributeMaxDynamicSharedMemorySize,
-                               (int)q8_lds_bytes(16)), "p0_open: gemv");
-  return P0_OK;
-}
-
-// q8g64s.t64: one workgroup per (64-row tile, split), gemv_q8.hip
-static int launch_q8(GemvP& p, int M, const char* op) {
+// q8g64s.t64 at M = 1: one workgroup per (64-row tile, split), gemv_q8.hip
+static int launch_q8(GemvP& p, const char* op) {
   // q8_gemv1_kernel: 16 waves per (tile, split), for splits of 1024-3072 k (16-48 groups; a split of 4 groups, the
   // E2B pleg projection's 256 k, runs faster on the 4-wave kernel: 3.9 against 4.9 us)
-  if (M == 1 && p.kPer >= 1024 && p.kPer <= 3072) {
+  if (p.kPer >= 1024 && p.kPer <= 3072) {
     // K-slices across workgroups (p.nks) when the tiles and splits leave most CUs idle: up to ~192 workgroups, at
     // least 8 groups (512 k) a slice (measured at the E2B 8-bit shapes: 6.2-9.3 us per launch against 6.9-10.9 with
     // one workgroup per split; p0_gemv_tune knob 5 sets the count)
@@ -559,16 +549,19 @@ static int launch_q8(GemvP& p, int M, const char* op) {
     P0_LAUNCHED(op);
     return P0_OK;
   }
-  q8_kernel_t k = q8_kernel(M);
-  const size_t lds = q8_lds_bytes(M);
-  hipLaunchKernelGGL(k, dim3((unsigned)p.NT, (unsigned)p.nsplit), dim3(256), lds, ctx().cur, p);
+  hipLaunchKernelGGL(q8_kernel(), dim3((unsigned)p.NT, (unsigned)p.nsplit), dim3(256), q8_lds_bytes(), ctx().cur, p);
   P0_LAUNCHED(op);
   return P0_OK;
 }
 
 static int launch(GemvP& p, int M, const char* op) {
   ChainBuild* cb = g_chain;
-  if (p.enc == P0_ENC_Q8G64S_T64 && !cb) return launch_q8(p, M, op);
+  if (!cb && M >= 2 && (p.enc == P0_ENC_Q8G64S_T64 || M >= g_mf_min_m)) {   // the matrix-core GEMV-M
+    launch_gemvm(p, ctx().cur);
+    P0_LAUNCHED(op);
+    return P0_OK;
+  }
+  if (p.enc == P0_ENC_Q8G64S_T64 && !cb) return launch_q8(p, op);
   if (cb && cb->M == 0) {   // the chain's first GEMV fixes M and the workgroup shape
     cb->M = M;
     cb->W = M == 1 ? g_chain_waves : 8;
@@ -607,13 +600,13 @@ static int launch(GemvP& p, int M, const char* op) {
   p.part = ctx().part;
   p.cnt = ctx().counters;
   p.coh = 0;   // chains: set for the whole chain by p0_chain_end
-  p.mf = !cb && M >= 2 && M >= g_mf_min_m;   // must agree with plan()'s LDS layout
+  p.mf = 0;      // pipelined chains: set by p0_chain_end
   if (cb) {
     cb->ops.push_back(p);
     if (pl.lds > cb->lds) cb->lds = pl.lds;
     return P0_OK;
   }
-  gemv_kernel_t k = pick(M, pl.mode + (p.mf ? 3 : 0));
+  gemv_kernel_t k = pick(M, pl.mode);
   dim3 grid((unsigned)pl.ntb, (unsigned)(p.nsplit * pl.nks));
   hipLaunchKernelGGL(k, grid, dim3(64 * pl.waves), pl.lds, ctx().cur, p);
   P0_LAUNCHED(op);

@@ -76,7 +76,7 @@ struct GemvP {
   // op reads or writes waits for op i - wback's completion flags before it writes them: 1 if op i - 1 reads them, 2 if
   // only ops before i - 1 do, 0 if none does
   int wback;
-  int mf;             // M >= 2: the MFMA arithmetic (standalone: gemv_item; pipelined chains: the slots), else fp32 VALU
+  int mf;             // pipelined chains, M >= 2: the slots' arithmetic on MFMA, else fp32 VALU
   // pipelined M > 1 chains on the matrix cores: an op whose input is one split of the previous op's output takes its x'
   // already staged by that op (stgIn), which writes, besides its outputs, the next op's prologue values as the matrix
   // cores' fp16 hi / lo A operands and the group sums as 16-row halves (stgOut, layout at stg_half_at): the consumer
@@ -264,7 +264,7 @@ struct Rec {
   uint32_t sm;
 };
 
-// ---- GEMV-M on MFMA (standalone launches, M >= 2). Per q4 group and 16 weight rows, two v_mfma_f32_16x16x32_f16
+// ---- the matrix-core arithmetic of chains with M > 1 rows (and, with a scale per row, of gemvm.hip). Per q4 group and 16 weight rows, two v_mfma_f32_16x16x32_f16
 // compute D[m][n] = 2^8 sum_k x'[m][k] q[n][k]: the A operand holds 2^8 x' split into fp16 hi + lo (2^8 x' = hi + lo to
 // 2^-22), the B operand the codes as exact fp16 values q (even k) and 16 q (odd k, whose x' carry the 1/16). Every
 // operand is a normal fp16 number: the codes come out of a code word as 1024 + q (the masked nibbles with the exponent
@@ -273,7 +273,7 @@ struct Rec {
 // ~3e-7 to 3.4e-6 relative L2 off the M = 1 row on MI355X: the matrix cores do not take fp16 subnormals at full
 // precision.)
 // Rounding: these rows are not bit-identical to the fp32 VALU path's (which p0_q4_gemv and the chain kernels use);
-// they agree to ~3e-7 relative L2. The VALU path for every M is p0_gemv_tune knob 4 = 17.
+// they agree to ~3e-7 relative L2. Standalone launches stay on the VALU with p0_gemv_tune knob 4 = 17.
 // Lane l holds D[4 (l / 16) + i][l % 16]: one weight row per lane, so each lane applies its row's scale and min
 // (2^-8 s D + m sum x') in fp32.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -326,19 +326,6 @@ __device__ __forceinline__ bool stage_x_mf(const GemvP& p, int g0, int g1, int g
   return bad;
 }
 
-// one group's records of one 64-row tile as loaded: lane = row, its four code words and its scale/min word (two loads
-// per lane; quarter_transpose turns them into the MFMA B layout)
-struct RecM {
-  u32x4 q;
-  uint32_t sm;
-};
-__device__ __forceinline__ RecM load_rec_mf(const GemvP& p, int64_t tile, int g, int lane) {
-  const uint8_t* rec = p.w + (int64_t)__builtin_amdgcn_readfirstlane((int)(tile * p.wG + g)) * 1280;
-  RecM r;
-  r.q = *P0_GLOBAL(const u32x4, rec + lane * 16);
-  r.sm = *P0_GLOBAL(const uint32_t, rec + 1024 + lane * 4);
-  return r;
-}
 // w[j] at lane 16 Q + i (Q the lane's 16-lane row) holds word j of weight row 16 Q + i; afterwards w[b] at lane 16 q + i
 // holds word q of weight row 16 b + i, the B layout of block b (lane l: word l / 16 of row 16 b + l % 16). A 4 x 4
 // transpose of (lane row, word) with the gfx950 lane swaps: permlane32_swap exchanges lanes 32-63 of its first operand
@@ -467,7 +454,7 @@ __device__ __forceinline__ float epilogue(const P& p, int split, int m, int tile
 // first poll then returns behind those loads (a wave's loads complete in order), which costs nothing when the wait is
 // longer than the loads' latency, and a wave that issued them after the wait would hold the whole workgroup at the
 // prologue's barrier for a full HBM latency.
-template <int M, int MODE, bool CHAIN, class Ready, bool MFK = false>
+template <int M, int MODE, bool CHAIN, class Ready>
 __device__ __forceinline__ bool gemv_item(const GemvP& p, int bx, int by, float* smem, int* s_last, Ready&& ready) {
   constexpr int T = MODE == 0 ? 1 : 2;
   constexpr int TPW = MODE == 1 ? 2 : 1;   // distinct output tiles per wave
@@ -483,13 +470,9 @@ __device__ __forceinline__ bool gemv_item(const GemvP& p, int bx, int by, float*
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kwv = wv % p.kw, tw = wv / p.kw;
   const int KL = p.gps * 32;
-  // MF: GEMV-M on MFMA (stage_x_mf); the fp32 VALU path stays for a workgroup whose x' is too large for fp16
-  constexpr bool MF = MFK && !CHAIN && M >= 2;
-  constexpr bool mf = MF;
-  const int XS = mf && M < 16 ? 16 : M;   // group-sum entries per group (MF: a 16-row A operand)
-  float* xs = smem;                    // [M][KL]   x' of the slice, odd k scaled 1/16 (MF: the A operands, same size)
-  float* xsum = smem + M * KL;         // [M][gps]  group sums of x' (MF: [gps][16])
-  float* red = xsum + XS * p.gps;      // [waves][T][64] in-workgroup reduction
+  float* xs = smem;                    // [M][KL]   x' of the slice, odd k scaled 1/16
+  float* xsum = smem + M * KL;         // [M][gps]  group sums of x'
+  float* red = xsum + M * p.gps;       // [waves][T][64] in-workgroup reduction
 
   const int split = by / p.nks, ks = by - split * p.nks;
   const int k0s = split * p.kPer, k1s = min(p.K, k0s + p.kPer);
@@ -515,100 +498,8 @@ __device__ __forceinline__ bool gemv_item(const GemvP& p, int bx, int by, float*
   const bool streams = active && wg0 < wg1;
 
   // ---- the share's first chunk is issued before the input is read: its latency overlaps the wait and the prologue
-  if (mf && tid == 0) *s_last = 0;   // MF: the "x' too large" flag until the split-K arrival reuses the word
   __syncthreads();   // the previous item of this workgroup is done with the LDS
   float acc[T][M];
-  bool mfd = false;   // MF: acc filled by the MFMA path
-  if constexpr (MF) {
-    constexpr int DM = 4;   // groups per chunk of records (8 registers per group and tile)
-    RecM m0[DM][T];
-    if (streams) {
-#pragma unroll
-      for (int i = 0; i < DM; ++i)
-#pragma unroll
-        for (int t = 0; t < T; ++t) m0[i][t] = load_rec_mf(p, tl(t), min(wg0 + i, glast), lane);
-    }
-    if (stage_x_mf<M, false, (M < 16 ? 16 : M)>(p, g0, g1, p.gps, (_Float16*)xs, xsum, tid, blockDim.x)) *s_last = 1;
-    __syncthreads();
-    if (*s_last == 0) {
-      float am[T][4][4];   // [tile][16-row block][i]: rows 16 b + lane % 16, x row 4 (lane / 16) + i
-#pragma unroll
-      for (int t = 0; t < T; ++t)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) am[t][b][i] = 0.0f;
-      const _Float16* xh = (const _Float16*)xs;
-      const int arow = min(lane & 15, M - 1), aw = lane >> 4;
-      auto consume_mf = [&](const RecM (&cur)[T], int g) {
-        const int gl = g - g0;
-        const half8_t* ap = (const half8_t*)(xh + (((gl * 4 + aw) * 2) * M + arow) * 8);
-        // rows >= M read row M - 1 (finite); their D rows are never used
-        const half8_t ahi = ap[0], alo = ap[M];
-        const f4_t sx = *(const f4_t*)(xsum + gl * 16 + 4 * aw);
-#pragma unroll
-        for (int t = 0; t < T; ++t) {
-          uint32_t qb[4] = {cur[t].q.x, cur[t].q.y, cur[t].q.z, cur[t].q.w};
-          uint32_t sb[4] = {cur[t].sm, cur[t].sm, cur[t].sm, cur[t].sm};
-          quarter_transpose(qb);
-          quarter_transpose(sb);
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const half8_t bq = codes_b(qb[b]);
-            f4_t d = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bq, f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bq, d, 0, 0, 0);
-            const float s8 = h2f_lo(sb[b]) * kMfDeq, mn = h2f_hi(sb[b]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) am[t][b][i] = __builtin_fmaf(s8, d[i], __builtin_fmaf(mn, sx[i], am[t][b][i]));
-          }
-        }
-      };
-      if (streams) {
-#pragma unroll
-        for (int i = 0; i < DM; ++i)
-          if (wg0 + i < wg1) consume_mf(m0[i], wg0 + i);
-        for (int c0 = wg0 + DM; c0 < wg1; c0 += DM) {
-          RecM r[DM][T];
-#pragma unroll
-          for (int i = 0; i < DM; ++i)
-#pragma unroll
-            for (int t = 0; t < T; ++t) r[i][t] = load_rec_mf(p, tl(t), min(c0 + i, glast), lane);
-#pragma unroll
-          for (int i = 0; i < DM; ++i)
-            if (c0 + i < wg1) consume_mf(r[i], c0 + i);
-        }
-      }
-      // back to one weight row per lane (acc[t][m] at lane = row) through this wave's reduction row: x row m lives in
-      // the 16 lanes l / 16 == m / 4, element m % 4, for rows 16 b + l % 16. Lanes hand values to other lanes here, so
-      // a wavefront fence on each side keeps the compiler from moving a read above other lanes' writes (the LDS itself
-      // serves one wave's accesses in order)
-      auto wave_sync = [] {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-      };
-#pragma unroll
-      for (int t = 0; t < T; ++t) {
-        float* tr = red + (wv * T + t) * 64;
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-          wave_sync();
-          if ((lane >> 4) == (m >> 2)) {
-#pragma unroll
-            for (int b = 0; b < 4; ++b) tr[16 * b + (lane & 15)] = am[t][b][m & 3];
-          }
-          wave_sync();
-          acc[t][m] = tr[lane];
-        }
-      }
-      mfd = true;
-    } else {
-      __syncthreads();   // x' too large for fp16: this workgroup stages fp32 x' and takes the VALU path
-      stage_x<M, false>(p, g0, g1, p.gps, xs, xsum);
-      __syncthreads();
-    }
-  }
-  if (!mfd) {
   Rec r0[D][T];
   if (streams) {
 #pragma unroll
@@ -619,11 +510,9 @@ __device__ __forceinline__ bool gemv_item(const GemvP& p, int bx, int by, float*
   if (!ready()) return false;
 
   // ---- prologue: x'[m][k] for the workgroup's K-slice -> LDS (odd k scaled 1/16), and the per-group sums of x'
-  if (!mf) {
-    if (coh_in) stage_x<M, true>(p, g0, g1, p.gps, xs, xsum);
-    else stage_x<M, false>(p, g0, g1, p.gps, xs, xsum);
-    __syncthreads();
-  }
+  if (coh_in) stage_x<M, true>(p, g0, g1, p.gps, xs, xsum);
+  else stage_x<M, false>(p, g0, g1, p.gps, xs, xsum);
+  __syncthreads();
 
   // ---- stream the records of the wave's share
 #pragma unroll
@@ -666,7 +555,6 @@ __device__ __forceinline__ bool gemv_item(const GemvP& p, int bx, int by, float*
         if (c0 + i < wg1) consume(r[i], c0 + i);
     }
   }
-  }   // !mfd
 
   // ---- the kw waves of a slot: sum their shares in wave order into wave kwv == 0. The reads are unrolled to the
   // largest kw (the workgroup's wave count) with clamped indices, so they issue back to back and wait once; the
@@ -925,15 +813,6 @@ __global__ __launch_bounds__(M <= 2 ? 1024 : 512) void q4_gemv_kernel(GemvP p) {
   gemv_item<M, MODE, false>(p, blockIdx.x, blockIdx.y, smem, &s_last, [] { return true; });
 }
 
-// the same GEMV-M on the matrix cores (M >= 2; the host sends p.mf calls here, with at most 8 waves per workgroup)
-template <int M, int MODE>
-__global__ __launch_bounds__(512) void q4_gemv_mf_kernel(GemvP p) {
-  extern __shared__ __attribute__((aligned(16))) float smem[];
-  __shared__ int s_last;
-  auto ready = [] { return true; };
-  gemv_item<M, MODE, false, decltype(ready)&, true>(p, blockIdx.x, blockIdx.y, smem, &s_last, ready);
-}
-
 // ---- the chain executor: a recorded sequence of GEMV ops in ONE persistent launch (the analogue of the reference's
 // per-token command buffer, engine/llm/drunner.js:1-8). Op i may read what ops < i wrote, so its items wait until op
 // i - 1 has written all of its outputs; each workgroup issues its first item's weight loads BEFORE that wait, so the
@@ -1058,12 +937,7 @@ typedef void (*gemv_kernel_t)(GemvP);
 typedef void (*chain_kernel_t)(const GemvP*, int, unsigned*, int);
 
 template <int M>
-gemv_kernel_t pick_m(int mode) {   // modes 3..5: modes 0..2 on the matrix cores (M >= 2)
-  if constexpr (M >= 2) {
-    if (mode == 3) return q4_gemv_mf_kernel<M, 0>;
-    if (mode == 4) return q4_gemv_mf_kernel<M, 1>;
-    if (mode == 5) return q4_gemv_mf_kernel<M, 2>;
-  }
+gemv_kernel_t pick_m(int mode) {
   if (mode == 0) return q4_gemv_kernel<M, 0>;
   if (mode == 1) return q4_gemv_kernel<M, 1>;
   return q4_gemv_kernel<M, 2>;
@@ -1075,12 +949,12 @@ chain_kernel_t pick_chain_m(int W) {   // 16-wave chain workgroups for M = 1, 8-
   return q4_gemv_chain_kernel<M, 8>;
 }
 
-// the q8g64s.t64 GEMV (gemv_q8.hip): the kernel for M rows and its LDS bytes
+// the q8g64s.t64 GEMV (M = 1, gemv_q8.hip): the kernels and their LDS bytes
 typedef void (*q8_kernel_t)(GemvP);
-q8_kernel_t q8_kernel(int M);
+q8_kernel_t q8_kernel();
 q8_kernel_t q8_gemv1(bool geglu);   // M = 1, splits of at most 3072 k: 16 waves, the records in flight together
 size_t q8_gemv1_lds_bytes();
-size_t q8_lds_bytes(int M);
+size_t q8_lds_bytes();
 
 // the pipelined chain (chain_pipe.hip) for M <= pipe_max_m() rows of x: its kernels and their shape
 chain_kernel_t pipe_chain_kernel(int M, bool q8);   // q8 (M = 1 only): the instantiation that also runs q8 ops

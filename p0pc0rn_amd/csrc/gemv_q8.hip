@@ -1,6 +1,6 @@
-// gemv_q8.hip - the q8g64s.t64 GEMV (M = 1, gemv) and GEMV-M (M <= 16, gemvM) on gfx950: the reference's other weight
-// encoding on the same call surface (engine/llm/lops.js:74-80, engine/llm/lops_spec.js:165), with the same prologues,
-// epilogues and split semantics as the q4 kernels (gemv_kernels.hpp).
+// gemv_q8.hip - the q8g64s.t64 GEMV (M = 1) on gfx950: the reference's other weight encoding on the same call surface
+// (engine/llm/lops.js:74-80), with the same prologues, epilogues and split semantics as the q4 kernels
+// (gemv_kernels.hpp). Its GEMV-M (2-16 rows) is in gemvm.hip.
 //
 // Data layout (packQ8, engine/kcheck.js:39-52): a weight W[N][K] is a sequence of 4224-byte records, record (tile, g)
 // = rows 64 tile .. + 63, k = 64 g .. + 63, tile-major. Bytes [64 r, 64 r + 64) are row r's 64 signed codes in k order;
@@ -20,19 +20,15 @@ constexpr int kQ8Waves = 4, kQ8Threads = 64 * kQ8Waves, kQ8Chunk = 1024, kQ8CG =
 // the M = 1 kernel: 16 waves, 2 groups per wave and round, splits of at most 3072 k
 constexpr int kQ81Waves = 16, kQ81Threads = 64 * kQ81Waves, kQ81G = 2, kQ81MaxK = 3072;
 
-size_t q8_lds_bytes(int M) {   // x' chunk, group sums, and the cross-wave reduction [wave][tile][m][lane]
-  return (size_t)M * (kQ8Chunk + kQ8CG) * sizeof(float) + (size_t)kQ8Waves * 2 * M * 64 * sizeof(float);
+size_t q8_lds_bytes() {   // x' chunk, group sums, and the cross-wave reduction [wave][tile][lane]
+  return (kQ8Chunk + kQ8CG + kQ8Waves * 2 * 64) * sizeof(float);
 }
 
-// MT: the compile-time row count (1), or 0 = p.mrows rows (at most 16)
-template <int MT>
 __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
-  constexpr int MM = MT ? MT : 16;
-  const int M = MT ? MT : p.mrows;
   extern __shared__ __attribute__((aligned(16))) float smem[];
-  float* xs = smem;                           // [M][kQ8Chunk]
-  float* xsum = xs + M * kQ8Chunk;            // [M][kQ8CG]
-  float* red = xsum + M * kQ8CG;              // [wave][T][M][64]
+  float* xs = smem;                           // [kQ8Chunk]
+  float* xsum = xs + kQ8Chunk;                // [kQ8CG]
+  float* red = xsum + kQ8CG;                  // [wave][T][64]
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const bool pair = p.epi == P0_EPI_GEGLU;
   const int T = pair ? 2 : 1;
@@ -40,25 +36,16 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
   const int64_t tiles[2] = {tile0, tile0 + (pair ? p.NT : 0)};
   const int k0s = split * p.kPer, k1s = min(p.K, k0s + p.kPer);
 
-  float acc[2][MM];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int m = 0; m < MM; ++m) acc[t][m] = 0.0f;
-
+  float acc[2] = {0.0f, 0.0f};
   for (int c0 = k0s; c0 < k1s; c0 += kQ8Chunk) {
     const int c1 = min(k1s, c0 + kQ8Chunk), ng = (c1 - c0) >> 6;
     __syncthreads();   // the previous chunk's x' is no longer read
-    for (int i = tid; i < M * kQ8Chunk; i += kQ8Threads) {
-      const int m = i / kQ8Chunk, kl = i - m * kQ8Chunk;
-      xs[i] = c0 + kl < c1 ? prologue<false>(p, m, c0 + kl) : 0.0f;
-    }
+    for (int i = tid; i < kQ8Chunk; i += kQ8Threads) xs[i] = c0 + i < c1 ? prologue<false>(p, 0, c0 + i) : 0.0f;
     __syncthreads();
-    for (int i = tid; i < M * kQ8CG; i += kQ8Threads) {   // group sums in k order
-      const int m = i / kQ8CG, gl = i - m * kQ8CG;
+    if (tid < kQ8CG) {   // group sums in k order
       float s = 0.0f;
-      for (int j = 0; j < 64; ++j) s += xs[m * kQ8Chunk + gl * 64 + j];
-      xsum[i] = s;
+      for (int j = 0; j < 64; ++j) s += xs[tid * 64 + j];
+      xsum[tid] = s;
     }
     __syncthreads();
     for (int gl = wv; gl < ng; gl += kQ8Waves) {
@@ -72,9 +59,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
         for (int j = 0; j < 4; ++j) q[j] = *P0_GLOBAL(const u32x4, rec + lane * 64 + j * 16);
         const uint32_t sw = *P0_GLOBAL(const uint32_t, rec + 4096 + (lane & ~1) * 2);
         const float s = (lane & 1) ? h2f_hi(sw) : h2f_lo(sw);
-        float d[MM];
-#pragma unroll
-        for (int m = 0; m < MM; ++m) d[m] = 0.0f;
+        float d = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const uint32_t wd[4] = {q[j].x ^ 0x80808080u, q[j].y ^ 0x80808080u, q[j].z ^ 0x80808080u, q[j].w ^ 0x80808080u};
@@ -82,20 +67,11 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
           for (int e = 0; e < 4; ++e) {
             const float b0 = (float)(wd[e] & 0xFFu), b1 = (float)((wd[e] >> 8) & 0xFFu);
             const float b2 = (float)((wd[e] >> 16) & 0xFFu), b3 = (float)(wd[e] >> 24);
-            const int kk = gl * 64 + j * 16 + e * 4;
-#pragma unroll
-            for (int m = 0; m < MM; ++m) {
-              if (m >= M) break;
-              const float4 x4 = *(const float4*)(xs + m * kQ8Chunk + kk);
-              d[m] = __builtin_fmaf(b0, x4.x, __builtin_fmaf(b1, x4.y, __builtin_fmaf(b2, x4.z, __builtin_fmaf(b3, x4.w, d[m]))));
-            }
+            const float4 x4 = *(const float4*)(xs + gl * 64 + j * 16 + e * 4);
+            d = __builtin_fmaf(b0, x4.x, __builtin_fmaf(b1, x4.y, __builtin_fmaf(b2, x4.z, __builtin_fmaf(b3, x4.w, d))));
           }
         }
-#pragma unroll
-        for (int m = 0; m < MM; ++m) {
-          if (m >= M) break;
-          acc[t][m] = __builtin_fmaf(s, d[m] - 128.0f * xsum[m * kQ8CG + gl], acc[t][m]);
-        }
+        acc[t] = __builtin_fmaf(s, d - 128.0f * xsum[gl], acc[t]);
       }
     }
   }
@@ -104,23 +80,19 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
   __syncthreads();
 #pragma unroll
   for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int m = 0; m < MM; ++m)
-      if (t < T && m < M) red[((wv * 2 + t) * M + m) * 64 + lane] = acc[t][m];
+    if (t < T) red[(wv * 2 + t) * 64 + lane] = acc[t];
   __syncthreads();
   if (wv != 0) return;
-  for (int m = 0; m < M; ++m) {
-    float tot[2] = {0.0f, 0.0f};
+  float tot[2] = {0.0f, 0.0f};
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      if (t >= T) break;
-      float v = red[((0 * 2 + t) * M + m) * 64 + lane];
+  for (int t = 0; t < 2; ++t) {
+    if (t >= T) break;
+    float v = red[t * 64 + lane];
 #pragma unroll
-      for (int w = 1; w < kQ8Waves; ++w) v += red[((w * 2 + t) * M + m) * 64 + lane];
-      tot[t] = v;
-    }
-    epilogue<false>(p, split, m, tile0, lane, tot[0], tot[1]);
+    for (int w = 1; w < kQ8Waves; ++w) v += red[(w * 2 + t) * 64 + lane];
+    tot[t] = v;
   }
+  epilogue<false>(p, split, 0, tile0, lane, tot[0], tot[1]);
 }
 
 // M = 1 (gemv, the decode case): a workgroup of 16 waves per (64-row tile, split), every wave's record loads issued
@@ -246,7 +218,7 @@ __global__ __launch_bounds__(kQ81Threads) void q8_gemv1_kernel(GemvP p) {
   epilogue<false>(p, split, 0, tile0, lane, tot[0], tot[1]);
 }
 
-q8_kernel_t q8_kernel(int M) { return M == 1 ? q8_gemv_kernel<1> : q8_gemv_kernel<0>; }
+q8_kernel_t q8_kernel() { return q8_gemv_kernel; }
 q8_kernel_t q8_gemv1(bool geglu) { return geglu ? q8_gemv1_kernel<2> : q8_gemv1_kernel<1>; }
 size_t q8_gemv1_lds_bytes() { return (kQ81MaxK + kQ81MaxK / 64 + kQ81Waves * 2 * 64) * sizeof(float); }
 

@@ -303,3 +303,53 @@ def test_gemvM_large_activations_keep_fp32(dev, mf, M):
     for m in range(M):
         c.x[m * 8192 + 4096: m * 8192 + 4096 + 7] = np.float32([400.0, -900.0, 330.0, 1.0e5, -3.5e3, 600.0, 2.0e4])
     c.check(f"gemvM M={M} large activations ({mf})")
+
+
+@pytest.mark.parametrize("M,N,K,pro,epi,kPer", [
+    (2, 64, 32, "raw", "store", 0),             # one group: one wave of eight has work
+    (3, 128, 5 * 32, "rms", "geglu", 0),        # a quad of groups with three of them past the end
+    (16, 192, 37 * 32, "rms", "store", 0),      # a second quad for two waves, one group in the last
+    (5, 64, 2048, "rms", "softcap", 0),         # every wave full
+    (4, 128, 4000, "raw", "store", 0),          # several passes of 2048 k in one split
+    (6, 64, 2080, "rms", "geglu", 0),           # a second pass of one group
+    (7, 320, 4128, "raw", "store", 2048),       # kPer splits, the last of one group
+    (5, 4160, 96, "raw", "store", 0),           # 260 blocks of 16 rows: two to an item
+    (2, 8256, 64, "rms", "store", 0),           # 516: four to an item
+    (2, 16448, 64, "rms", "store", 0),          # more items than workgroups
+    (9, 16512, 64, "raw", "softcap", 0),
+    (3, 16448, 64, "pleg", "geglu", 0),
+])
+def test_gemvM_matrix_core_shapes(dev, M, N, K, pro, epi, kPer):
+    """gemvm.hip where its pieces end: quads of groups, passes, items of 1, 2 and 4 blocks, several items a workgroup;
+    x rows and weights at 4-byte alignment, rows of y apart. The file's fp32 bar (the split of x' keeps 22 bits)"""
+    Case(M, N, K, pro, epi, kPer=kPer, seed=80 + M, w_off=4, rowB=3 if pro != "pleg" else 0, ldx=K + 5, ldm=N + 7,
+         gemvM=True).check(f"gemvM M={M} {N}x{K} {pro} {epi}")
+
+
+@pytest.mark.parametrize("scale", [1e-30, 1e-3, 1e4, 1e30])
+def test_gemvM_row_scales(dev, scale):
+    """each x row has a power-of-two scale of its own: rows many decades apart in one call keep the fp32 bar"""
+    c = Case(4, 128, 1024, "raw", "store", seed=95, gemvM=True)
+    for m, f in enumerate((1.0, scale, 1.0 / scale, 3.0)):
+        c.x[m * 1024:(m + 1) * 1024] *= np.float32(f)
+    yo, _ = c.run_oracle()
+    yg, _ = c.run_gpu()
+    for m in range(4):
+        _check(yg[m * 128:(m + 1) * 128], yo[m * 128:(m + 1) * 128], f"gemvM row {m}, scale {scale}")
+
+
+def test_gemvM_infinities_and_nan_keep_to_their_row(dev):
+    """rows with an infinity or a NaN are infinite or NaN where the oracle's are, and leave the other rows alone"""
+    M, N, K = 5, 128, 2048
+    c = Case(M, N, K, "rms", "store", seed=96, gemvM=True)
+    c.x[1 * K + 700] = np.inf
+    c.x[2 * K + 3] = np.nan
+    c.x[3 * K + 2047] = -np.inf
+    yo, _ = c.run_oracle()
+    yg, _ = c.run_gpu()
+    for m in range(M):
+        o, g = yo[m * N:(m + 1) * N], yg[m * N:(m + 1) * N]
+        if m in (0, 4):
+            _check(g, o, f"gemvM row {m} beside infinite rows")
+        else:
+            assert not np.isfinite(o).any() and not np.isfinite(g).any(), m

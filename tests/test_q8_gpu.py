@@ -288,3 +288,29 @@ def test_q8_ops_join_only_pipelined_chains(dev):
         capi.chain_tune(4, old)
     for v in (wb, xb, yb):
         v.free()
+
+
+@pytest.mark.parametrize("M,N,K,kPer,epi", [(2, 64, 64, 0, "store"), (16, 192, 9 * 64, 0, "geglu"), (5, 128, 2112, 0, "geglu"),
+                                            (7, 320, 4160, 2048, "store"), (5, 4160, 128, 0, "store"),
+                                            (3, 16448, 64, 0, "store")])
+def test_q8_gemvM_shapes(dev, M, N, K, kPer, epi):
+    """the q8 GEMV-M where its pieces end (one group, one past eight, a second pass of one group, kPer splits, items of 1,
+    2 and 4 blocks, several items a workgroup), rms prologue, x and weights at 4-byte alignment, rows of y apart"""
+    rows, ldx, ldm, ns = (2 * N if epi == "geglu" else N), K + 3, N + 5, (-(-K // kPer) if kPer else 1)
+    w = np.concatenate([np.zeros(4, np.uint8), np.asarray(_q8(rows, K, N + K)).view(np.uint8).ravel()])
+    x, nw = O.randn(M * ldx + 8, 73), nw_of(K)
+    st = (0.5 + O.rng_uniform(9, 2 * M)).astype(np.float32)
+    f = dict(w_enc=2, w_off=4, w_rows=rows, w_cols=K, x_rowB=1, x_ldx=ldx, M=M, N=N, K=K, kPer=kPer, pro=capi.PRO["rms"],
+             epi=capi.EPI[epi], y_ldm=ldm, y_ldy=M * ldm, stat_off=1, stat_ld=2)
+    want = np.full(ns * M * ldm + 16, np.nan, np.float32)
+    host = dict(w=w, x=x, norm=nw, stat=st)
+    O.q4_gemvM(capi.gemvm_args(**f, **{k: v.ctypes.data for k, v in host.items()}, y=want.ctypes.data))
+    dv = {k: capi.to_device(v) for k, v in host.items()}
+    yb = capi.Buffer(want.nbytes).fill_u32(0x7FC00000)
+    assert capi.q4_gemvM(capi.gemvm_args(**f, **dv, y=yb)) == ns
+    got = yb.read(np.float32)
+    assert np.array_equal(np.isnan(got), np.isnan(want))   # exactly the rows of y
+    ok = ~np.isnan(want)
+    assert rel_l2(got[ok], want[ok]) <= 2e-5
+    for v in list(dv.values()) + [yb]:
+        v.free()
