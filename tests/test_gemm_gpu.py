@@ -240,3 +240,50 @@ def test_gemm_staging_rows_per_wave(dev, mode, M, K, pad):
         arrays.update(stats=st, pv=pv)
     want, got = run(f, arrays, np.float32, M * N)
     check(got, want, f"gemm staging {mode} {M}x{K}", 5e-5)
+
+
+_SMALL = [  # (M, N, K, first weight row, its columns before K, epilogue): edges of 128 x 128 tiles, 64-k steps, K slices
+    (1, 64, 32, 0, 0, "f32"), (127, 128, 96, 64, 32, "f16"), (129, 200, 1056, 0, 64, "f32"), (130, 131, 4128, 128, 0, "bias"),
+    (257, 448, 2048, 0, 0, "resadd"), (64, 384, 544, 0, 32, "swiglu"), (200, 130, 2080, 64, 0, "swiglu"),
+    (77, 384, 1088, 0, 0, "heads-inter"), (140, 640, 96, 0, 0, "heads-half"), (300, 128, 8192, 0, 0, "resadd"),
+]
+
+
+@pytest.mark.parametrize("M,N,K,wr0,wk0,epi", _SMALL)
+def test_gemm_small_tiles_against_large(dev, M, N, K, wr0, wk0, epi):
+    """calls of one or a few tiles run in 128 x 128 tiles with K cut into slices (gemm_n128.hip); the same call on a weight
+    at a 4-byte offset runs in 256 x 256 tiles (gemm.hip). Both sum the same fp16 operands in fp32: each is within the
+    oracle's bar, and they differ by the order of the sums only (2e-6 relative in fp32 over K <= 8192: sqrt(K) roundings
+    of 2^-24; one fp16 ulp where the output is fp16)"""
+    sw, heads = epi == "swiglu", epi.startswith("heads")
+    rows = -(-(wr0 + (N if not sw else N // 2)) // 64) * 64
+    wr1 = rows if sw else 0
+    rows *= 2 if sw else 1
+    Kw = wk0 + K + 32
+    w = O.pack_q4(np.clip(O.randn(rows * Kw, M + N, 0.05), -0.3, 0.3), rows, Kw)[0]
+    x = O.randn(M * (K + 8), 7).astype(np.float16)
+    f32 = epi in ("f32", "resadd")
+    dt, ncol = (np.float32 if f32 else np.float16), (N // 2 if sw else N)
+    f = dict(w_rows=rows, w_cols=Kw, M=M, N=N, K=K, x_ld=K + 8, wr0=wr0, wr1=wr1, wk0=wk0, x_mode=0,
+             epi=capi.GEPI["heads" if heads else epi], y_ld=ncol + 3, y_n0=1)
+    arrays, n_out = dict(x=x), M * (ncol + 3) + 16
+    if epi in ("bias", "resadd"):
+        arrays.update(ev=O.randn(N, 43), bv=O.randn(N, 44, 0.1)) if epi == "resadd" else arrays.update(ev=O.randn(N, 43))
+        f.update(res=1) if epi == "bias" else None
+    if sw:
+        arrays.update(bv=O.randn(2 * N, 45, 0.1))
+        f.update(bv_up=N, act=capi.ACT["silu"])
+    if heads:
+        H, Ltot = N // 128, M + 5
+        rope = np.stack([np.cos(np.arange(Ltot * 64) * 0.01), np.sin(np.arange(Ltot * 64) * 0.01)], -1).astype(np.float32)
+        arrays.update(ev=(1 + O.randn(256, 46, 0.1)).astype(np.float32), rope=rope)
+        f.update(heads_ltot=Ltot, heads_row_off=3, heads_hq=H // 2, heads_hkv=1, heads_rope=capi.ROPE[epi[6:]])
+        n_out = H * Ltot * 128 + 16
+    init = O.randn(n_out, 47)
+    shifted = np.concatenate([np.zeros(4, np.uint8), np.asarray(w).view(np.uint8).ravel()])
+    want, small = run(f, dict(arrays, w=w), dt, n_out, init=init)
+    _, large = run(dict(f, w_off=4), dict(arrays, w=shifted), dt, n_out, init=init)
+    check(small, want, f"gemm small tiles {epi} {M}x{N}x{K}", 1e-5 if f32 else 2e-3)
+    check(small, large, f"gemm small against large tiles {epi}", 2e-6 if f32 else 1e-3)
+    untouched = want == init.astype(dt)
+    assert np.array_equal(small[untouched], want[untouched])
