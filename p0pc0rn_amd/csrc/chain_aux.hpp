@@ -86,6 +86,81 @@ __device__ __forceinline__ float aux_tree256(float v, lds_f32* area, int tc, lds
 
 __device__ __forceinline__ float aux_rsqrt(float v) { return 1.0f / __builtin_sqrtf(v); }
 
+// the op's fields, read once through the constant address space at an address made uniform: scalar loads, all in flight
+// together. (Through the pointer as it arrives, in vector registers, every field was a vector load of its own where it was
+// used, behind the stores before it: most of a normadd's time in a chain.)
+struct AuxP {
+  int kind, amode;
+  const float* asrc; float* adst; float* ast; const float* aw;
+  int64_t arows, acols, ald, ac0, an, aldp, astOff, awOff;
+  float aeps, ascale;
+};
+__device__ __forceinline__ AuxP aux_fields(const GemvP* pp) {
+  const uint64_t a = (uint64_t)(uintptr_t)pp;
+  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                     (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32;
+  const auto* c = (const __attribute__((address_space(4))) GemvP*)u;
+  return AuxP{c->kind, c->amode, c->asrc, c->adst, c->ast, c->aw, c->arows, c->acols, c->ald, c->ac0, c->an, c->aldp, c->astOff,
+              c->awOff, c->aeps, c->ascale};
+}
+
+// normadd (engine/llm/lops.js:153-170) of rows of up to 2048 values over up to 4 partials, every normadd of a decode
+// layer: the partials, the residual and the norm weights are all in flight before the first is used, one memory round
+// trip instead of one per partial and pass. A function of its own, so that it saves few registers of its caller's. With
+// this and the scalar fields the two normadds of a layer cost a chained M = 1 token (30 layers) 6 us each, the flags before and after them included; 16 before.
+__host__ __device__ inline bool aux_normadd_fits(int64_t D, int64_t n) { return D <= kAuxBatch * 256 && n <= 4; }
+__device__ __noinline__ unsigned aux_normadd(const GemvP* pp, int b, int G, int tc, lds_f32* lds, lds_u32* ctr, unsigned gen) {
+#pragma clang fp contract(off)
+  const AuxP p = aux_fields(pp);
+  b = __builtin_amdgcn_readfirstlane(b);
+  G = __builtin_amdgcn_readfirstlane(G);
+  const int D = (int)p.acols;
+  int area = 0;   // the two tree areas alternate, so a tree's writes never meet a slower wave's reads of the one before
+  for (int64_t r = b; r < p.arows; r += G) {
+    const int64_t xb = r * D;
+    float t[kAuxBatch], xv[kAuxBatch], wv8[kAuxBatch], s = 0.0f, s2 = 0.0f;
+    const bool mine = tc < 256;
+    if (mine) {
+      float v[4][kAuxBatch];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (j < p.an)
+#pragma unroll
+          for (int u = 0; u < kAuxBatch; ++u)
+            v[j][u] = tc + u * 256 < D ? aux_ldf(p.asrc + j * p.aldp + xb + tc + u * 256) : 0.0f;
+      if (p.amode == 0)
+#pragma unroll
+        for (int u = 0; u < kAuxBatch; ++u) {
+          const bool in = tc + u * 256 < D;
+          xv[u] = in ? aux_ldf(p.adst + xb + tc + u * 256) : 0.0f;
+          wv8[u] = in ? aux_ldf(p.aw + p.awOff + tc + u * 256) : 0.0f;
+        }
+#pragma unroll
+      for (int u = 0; u < kAuxBatch; ++u) {
+        t[u] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j < p.an) t[u] = t[u] + v[j][u];
+        if (tc + u * 256 < D) s = s + t[u] * t[u];
+      }
+    }
+    const float rs = aux_rsqrt(aux_tree256(s, lds + area * 256, tc, ctr, gen) / (float)D + p.aeps);
+    area ^= 1;
+    if (mine)
+#pragma unroll
+      for (int u = 0; u < kAuxBatch; ++u) {
+        if (tc + u * 256 >= D) continue;
+        const float x = p.amode == 0 ? (xv[u] + t[u] * rs * wv8[u]) * p.ascale : t[u];
+        aux_stf(p.adst + xb + tc + u * 256, x);
+        s2 = s2 + x * x;
+      }
+    const float r2 = aux_tree256(s2, lds + area * 256, tc, ctr, gen);
+    area ^= 1;
+    if (tc == 0) aux_stf(p.ast + p.astOff + r, aux_rsqrt(r2 / (float)D + p.aeps));
+  }
+  return gen;
+}
+
 // aux op p in workgroup b of G, compute thread tc (0 .. 511); lds: kAuxLdsFloats floats of this workgroup's LDS, free
 // during the op; ctr / gen: the compute waves' barrier (aux_bar). The caller has waited for op i - 1 in every
 // workgroup, and waits for these stores (vmcnt) before it publishes the op. Not inlined: the chain kernels' GEMV code
@@ -93,7 +168,9 @@ __device__ __forceinline__ float aux_rsqrt(float v) { return 1.0f / __builtin_sq
 __device__ __noinline__ unsigned aux_run(const GemvP* pp, int b, int G, int tc, lds_f32* lds, lds_u32* ctr,
                                          unsigned gen) {
 #pragma clang fp contract(off)
-  const GemvP& p = *pp;
+  const AuxP p = aux_fields(pp);
+  b = __builtin_amdgcn_readfirstlane(b);
+  G = __builtin_amdgcn_readfirstlane(G);
   const int lane = tc & 63, wv = tc >> 6;
   if (p.kind == kOpCopy) {
     for (int64_t base = (int64_t)b * kAuxCopyWords; base < p.an; base += (int64_t)G * kAuxCopyWords) {
@@ -193,9 +270,10 @@ __device__ __noinline__ unsigned aux_run(const GemvP* pp, int b, int G, int tc, 
       }
       continue;
     }
-    // normadd, engine/llm/lops.js:153-170: the t sums are added again in the second pass (the same order, the same
-    // bits) instead of being kept in LDS
+    // normadd, engine/llm/lops.js:153-170
     const int64_t D = p.acols, xb = r * D;
+    // longer rows and more partials than aux_normadd's: the t sums are added again in the second pass (the same order, the
+    // same bits) instead of being kept
     // t of elements i0 + 256 u (u < kAuxBatch, those < D): the partials added in j order, a batch of loads per j
     auto tsum = [&](int64_t i0, float (&t)[kAuxBatch]) {
 #pragma unroll

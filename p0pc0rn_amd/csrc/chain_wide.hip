@@ -309,7 +309,10 @@ __global__ __launch_bounds__(64 * kPW) void q4_chain_wide_kernel(const GemvP* __
           abandon = true;
           break;
         }
-        gen = aux_run(&p, b, G, tc, (lds_f32*)red0, lctl + L::CtlBar, gen);
+        if (p.kind == kOpNormadd && aux_normadd_fits(p.acols, p.an))
+          gen = aux_normadd(&p, b, G, tc, (lds_f32*)red0, lctl + L::CtlBar, gen);
+        else
+          gen = aux_run(&p, b, G, tc, (lds_f32*)red0, lctl + L::CtlBar, gen);
         __builtin_amdgcn_s_waitcnt(0);
         cbar();
       }
