@@ -87,6 +87,35 @@ def test_aux_only_chain_matches_oracle(dev):
         b.free()
 
 
+@pytest.mark.parametrize("D,nsrc,M", [(4, 1, 1), (100, 4, 2), (2048, 1, 16), (2048, 4, 3), (2048, 5, 2), (2052, 4, 2)])
+def test_chain_normadd_sizes(dev, D, nsrc, M):
+    """a chained normadd's two forms on both sides of the rule (D <= 2048, at most 4 partials), bit for bit"""
+    ldp = M * D + 4
+    h = dict(t=O.randn(nsrc * ldp, 11, 0.3), w=(0.5 + O.rng_uniform(12, D)).astype(np.float32), x=O.randn(M * D, 13))
+    d = {k: capi.to_device(h[k]) for k in ("t", "w")}
+    xs, sts = [capi.Buffer(M * D * 4) for _ in range(2)], [capi.Buffer((M + 1) * 4).fill_u32(NAN) for _ in range(2)]
+    src = capi.to_device(h["x"])
+    nk = dict(t_n=nsrc, t_ld=ldp, w_off=0, st_off=1, D=D, M=M, eps=1e-6, scale=0.9)
+
+    def ops():
+        for mode in (0, 1):
+            capi.copy(src, 0, xs[mode], 0, M * D * 4)
+            capi.normadd(capi.normadd_args(t=d["t"], w=d["w"], x=xs[mode], st=sts[mode], mode=mode, **nk))
+
+    ch = capi.chain(ops)
+    ch.run()
+    assert ch.status() == 0
+    for mode in (0, 1):
+        xw, sw = h["x"].copy(), np.full(M + 1, np.nan, np.float32)
+        O.normadd(capi.normadd_args(t=h["t"].ctypes.data, w=h["w"].ctypes.data, x=xw.ctypes.data, st=sw.ctypes.data,
+                                    mode=mode, **nk))
+        assert np.array_equal(_bits(xs[mode].read(np.float32)), _bits(xw)), f"x, mode {mode}"
+        assert np.array_equal(_bits(sts[mode].read(np.float32)[1:]), _bits(sw[1:])), f"st, mode {mode}"
+    ch.free()
+    for b in list(d.values()) + xs + sts + [src]:
+        b.free()
+
+
 class TokenStep(MiniStep):
     """MiniStep as a whole decode token: after the layer ops, the rstd copy into the head's stat slot, the softcap
     head (rms, its rstd read from that slot), the argmax over its tile maxima and the copy of the result words into a
