@@ -215,7 +215,7 @@ int p0_q4_dequant(const void* w, int64_t w_off, int64_t N, int64_t K, float* out
  * knob 4: fewest x rows M from which a q4 gemvM call outside a chain runs on the matrix cores (default 2, i.e. every
  *         M > 1; 17: never, the fp32 VALU kernel). Knobs 0-3 plan the VALU kernel (M = 1 by default); the matrix-core
  *         kernel splits K over the waves of a workgroup only.
- * knob 5: K-slices per split of a q8g64s.t64 gemv (M = 1, splits of 1024-3072 k) across workgroups (default 0: planned,
+ * knob 5: K-slices per split of a q8g64s.t64 gemv (M = 1, splits of 2112-3072 k) across workgroups (default 0: planned,
  *         up to ~192 workgroups with at least 8 groups of 64 k a slice; a negative value restores the plan).
  * value <= 0 only queries (knob 5: value < 0 restores its plan). Returns the previous value, or -1 for an unknown
  * knob. */

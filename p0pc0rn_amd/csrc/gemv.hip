@@ -522,11 +522,11 @@ static bool plan_wide(std::vector<GemvP>& ops, int G) {
   return true;
 }
 
-// q8g64s.t64 at M = 1: one workgroup per (64-row tile, split), gemv_q8.hip
+// q8g64s.t64 at M = 1 in splits of more than 2048 k (smaller ones: gemv1.hip): one workgroup per (64-row tile, split),
+// gemv_q8.hip
 static int launch_q8(GemvP& p, const char* op) {
-  // q8_gemv1_kernel: 16 waves per (tile, split), for splits of 1024-3072 k (16-48 groups; a split of 4 groups, the
-  // E2B pleg projection's 256 k, runs faster on the 4-wave kernel: 3.9 against 4.9 us)
-  if (p.kPer >= 1024 && p.kPer <= 3072) {
+  // q8_gemv1_kernel: 16 waves per (tile, split), whose LDS holds at most 3072 k
+  if (p.kPer <= 3072) {
     // K-slices across workgroups (p.nks) when the tiles and splits leave most CUs idle: up to ~192 workgroups, at
     // least 8 groups (512 k) a slice (measured at the E2B 8-bit shapes: 6.2-9.3 us per launch against 6.9-10.9 with
     // one workgroup per split; p0_gemv_tune knob 5 sets the count)
@@ -558,6 +558,11 @@ static int launch(GemvP& p, int M, const char* op) {
   ChainBuild* cb = g_chain;
   if (!cb && M >= 2 && (p.enc == P0_ENC_Q8G64S_T64 || M >= g_mf_min_m)) {   // the matrix-core GEMV-M
     launch_gemvm(p, ctx().cur);
+    P0_LAUNCHED(op);
+    return P0_OK;
+  }
+  if (!cb && M == 1 && gemv1_takes(p)) {
+    launch_gemv1(p, ctx().cur);
     P0_LAUNCHED(op);
     return P0_OK;
   }

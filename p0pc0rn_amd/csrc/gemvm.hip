@@ -30,9 +30,6 @@
 
 namespace p0 {
 
-constexpr int kGmWaves = 8, kGmThreads = 64 * kGmWaves;
-constexpr int kGmPass = 2048;   // k per pass: 8 waves x 8 chunks of 32
-
 typedef uint32_t u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));
 
 // 8 codes (two words) of a q8 row as exact fp16 values: byte ^ 0x80 = q + 128 under the exponent of 1024, minus 1152
@@ -47,16 +44,6 @@ __device__ __forceinline__ half8_t codes_q8(uint32_t w0, uint32_t w1) {
   }
   return __builtin_bit_cast(half8_t, u);
 }
-
-// The kernel's arguments, offsets folded into the pointers: three cache lines, read at the start (the whole op
-// description, GemvP, is 500 bytes that a cold launch fetches line by line as they come up)
-struct GmP {
-  const uint8_t* w; const float* X; const float* ST; const float* NW; const float* EV;
-  int64_t wG, ldx, statLd, ldp, evLd;
-  int N, K, kPer, M, pro, nsrc, items, ipw, wgs;   // wgs: workgroups per split
-  int epi, NT; float cap;
-  float* Y; float* MX; int64_t ldy, ldm;
-};
 
 // One launch: grid (workgroups, splits); workgroup pos takes items [pos ipw, (pos + 1) ipw) of its split
 template <int ENC, int NBK, bool GEGLU, bool PLEG>
@@ -337,34 +324,16 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
 
 template <int ENC>
 static void launch_enc(const GemvP& p, hipStream_t s) {
-  // blocks of 16 weight rows over all splits, as many to an item (1, 2 or 4) as keep the items within one per CU (a CU
-  // holds one workgroup: the next one starts by splitting x' again); a geglu's gate and up block go together, a softcap
-  // needs its tile's 4. q8 5120 x 1536, 5 rows: 320 items of one block 13.5 us, 160 of two 8.8
-  const int geglu = p.epi == P0_EPI_GEGLU, rows16 = p.N / 16;
-  const int64_t blocks = (int64_t)rows16 * (geglu ? 2 : 1) * p.nsplit;
-  const int nbk = p.epi == P0_EPI_SOFTCAP || blocks > 512 ? 4 : blocks > 256 || geglu ? 2 : 1;
-  const int items = rows16 / (geglu ? nbk / 2 : nbk);
-  const int slots = 256 / (p.nsplit < 256 ? p.nsplit : 256);   // workgroups per split; more items than that are shared out
-  const int wgs = items < slots ? items : slots < 1 ? 1 : slots;
-  const int ipw = (items + wgs - 1) / wgs;
-  const dim3 grid((unsigned)((items + ipw - 1) / ipw), (unsigned)p.nsplit);
-  GmP g{};
-  g.w = p.w;
-  g.X = p.X + (p.pro == P0_PRO_PLEG ? 0 : p.rowB);   // pleg partials carry no row base
-  g.ST = p.ST + p.statOff;
-  g.NW = p.NW + p.nOff;
-  g.EV = p.EV + p.evOff;
-  g.wG = p.wG; g.ldx = p.ldx; g.statLd = p.statLd; g.ldp = p.ldp; g.evLd = p.evLd;
-  g.N = p.N; g.K = p.K; g.kPer = p.kPer; g.M = p.mrows; g.pro = p.pro; g.nsrc = p.nsrc;
-  g.items = items; g.ipw = ipw; g.wgs = (int)grid.x;
-  g.epi = p.epi; g.NT = p.NT; g.cap = p.cap;
-  g.Y = p.Y; g.MX = p.MX; g.ldy = p.ldy; g.ldm = p.ldm;
+  const GmPlan pl = gm_plan(p, 512);
+  const GmP& g = pl.args;
+  const bool geglu = p.epi == P0_EPI_GEGLU;
+  const int nbk = pl.nbk;
   const bool pleg = p.pro == P0_PRO_PLEG;
 #define P0_GM(NBK, GEGLU) (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true> : gemvm_kernel<ENC, NBK, GEGLU, false>)
   auto k = geglu ? (nbk == 4 ? P0_GM(4, true) : P0_GM(2, true))
                  : nbk == 4 ? P0_GM(4, false) : nbk == 2 ? P0_GM(2, false) : P0_GM(1, false);
 #undef P0_GM
-  hipLaunchKernelGGL(k, grid, dim3(kGmThreads), 0, s, g);
+  hipLaunchKernelGGL(k, pl.grid, dim3(kGmThreads), 0, s, g);
 }
 
 void launch_gemvm(const GemvP& p, hipStream_t s) {

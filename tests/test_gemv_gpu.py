@@ -326,6 +326,27 @@ def test_gemvM_matrix_core_shapes(dev, M, N, K, pro, epi, kPer):
          gemvM=True).check(f"gemvM M={M} {N}x{K} {pro} {epi}")
 
 
+@pytest.mark.parametrize("N,K,pro,epi,kPer", [
+    (64, 32, "raw", "store", 0),                # one group: one quarter of one wave has work
+    (128, 5 * 32, "rms", "geglu", 0),           # a second wave with one group of its quad
+    (192, 37 * 32, "sum", "store", 0),          # a second quad for two waves, one group in the last
+    (64, 2048, "rms", "softcap", 0),            # every wave full
+    (128, 2080, "raw", "store", 0),             # one group more than a split may hold there
+    (320, 4128, "raw", "store", 2048),          # kPer splits, the last of one group
+    (320, 4128, "pleg", "store", 1056),
+    (4160, 96, "raw", "store", 0),              # 260 blocks of 16 rows: two to an item
+    (16448, 64, "rms", "store", 0),             # more items than workgroups, an uneven share
+    (16448, 64, "pleg", "geglu", 0),
+    (16512, 64, "raw", "softcap", 0),
+    (65536, 32, "raw", "store", 0),             # the largest there, and one tile more
+    (65600, 32, "rms", "softcap", 0),
+])
+def test_gemv_one_row_shapes(dev, N, K, pro, epi, kPer):
+    """gemv1.hip where its pieces end, on both sides of its rule (kPer, tiles), x rows and weights at 4-byte alignment"""
+    Case(1, N, K, pro, epi, kPer=kPer, seed=70, w_off=4, rowB=3 if pro in ("raw", "rms") else 0, ldx=K + 5).check(
+        f"gemv {N}x{K} {pro} {epi}")
+
+
 @pytest.mark.parametrize("scale", [1e-30, 1e-3, 1e4, 1e30])
 def test_gemvM_row_scales(dev, scale):
     """each x row has a power-of-two scale of its own: rows many decades apart in one call keep the fp32 bar"""

@@ -77,6 +77,45 @@ def test_q8_k_slices_across_workgroups(dev, slices, pro, epi, K, kPer):
         capi.gemv_tune(5, old if old > 0 else -1)
 
 
+@pytest.mark.parametrize("N,K,pro,epi,kPer", [
+    (64, 64, "raw", "store", 0),                # one group: one wave has work
+    (128, 9 * 64, "rms", "geglu", 0),           # a second group for one wave
+    (192, 2048, "raw", "softcap", 0),           # every wave full
+    (320, 4160, "raw", "store", 2048),          # kPer splits, the last of one group
+    (4160, 128, "rms", "store", 0),             # 260 blocks of 16 rows: two to an item
+    (8256, 64, "rms", "geglu", 0),              # more items than workgroups, an uneven share
+    (8256, 64, "raw", "softcap", 0),
+    (128, 2112, "rms", "geglu", 0),             # splits that gemv_q8.hip takes
+    (128, 3072, "raw", "store", 0),
+])
+def test_q8_one_row_shapes(dev, N, K, pro, epi, kPer):
+    """gemv1.hip's q8 form where its pieces end, and the splits past its rule; the bar of the file's gemvM test"""
+    rows, nsplit = 2 * N if epi == "geglu" else N, -(-K // kPer) if kPer else 1
+    h = dict(w=_q8(rows, K, 61), x=O.randn(K + 3, 62), nw=nw_of(K), st=np.array([0, 0.7], np.float32),
+             mx=np.array([0, 0.7] * (N // 64 + 1), np.float32))
+    d = {k: capi.to_device(v) for k, v in h.items()}
+    want = np.full(nsplit * N, np.nan, np.float32)
+    yb = capi.Buffer(want.nbytes).fill_u32(0x7FC00000)
+
+    def args(b, y, at):
+        f = dict(w=at(b["w"]), w_enc=2, w_rows=rows, w_cols=K, x=at(b["x"]), x_rowB=3, N=N, K=K, kPer=kPer, pro=capi.PRO[pro],
+                 epi=capi.EPI[epi], y=y, mx=at(b["mx"]), cap=30.0)
+        if pro == "rms":
+            f.update(norm=at(b["nw"]), stat=at(b["st"]), stat_off=1)
+        return capi.gemv_args(**f)
+
+    O.q4_gemv(args(h, want.ctypes.data, lambda a: a.ctypes.data))
+    assert capi.q4_gemv(args(d, yb, lambda b: b)) == nsplit
+    got = yb.read(np.float32)
+    r = rel_l2(got, want)
+    print(f"q8 gemv {N}x{K} {pro} {epi}: rel_l2 {r:.3e}", flush=True)
+    assert np.all(np.isfinite(got)) and r <= 2e-5
+    if epi == "softcap":
+        assert np.allclose(d["mx"].read(np.float32)[0:N // 32:2], h["mx"][0:N // 32:2], rtol=1e-5, atol=1e-5)
+    for v in list(d.values()) + [yb]:
+        v.free()
+
+
 @pytest.mark.parametrize("M,epi", [(5, "store"), (16, "store"), (3, "softcap")])
 def test_q8_gemvM_matches_oracle(dev, M, epi):
     N, K = 256, 2048
