@@ -224,6 +224,59 @@ __global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T
   if (lane == 0) ST[stoff + m] = rsqrt_exact(r2 / (float)D + eps);
 }
 
+// The same for rows of at most 2048 values, 16-byte aligned, and few of them (a decode step's, a verify pass's): a wave per
+// chunk of 256, all of its loads in flight before the first sum; the chunks' squares meet in LDS, where every wave adds
+// them in chunk order, which is partial t's order. Per recorded launch 2048 values over 1 or 4 partials take 2.7 us (one
+// wave a row: 4.1), 256 rows 3.3; a decode token as a recording, 60 of them, 913 -> 870 us. More rows than CUs: a wave a row.
+constexpr int kNaWaves = 8, kNaThreads = 64 * kNaWaves;
+__global__ __launch_bounds__(kNaThreads) void normadd_few_kernel(const float* __restrict__ T, int64_t nsrc, int64_t ldp,
+                                                                 const float* __restrict__ W, int64_t woff, float* X,
+                                                                 float* __restrict__ ST, int64_t stoff, int D, float eps,
+                                                                 float scale, int mode) {
+  __shared__ __attribute__((aligned(16))) float sq[2][kNaWaves][kChunk];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i = wv * kChunk + 4 * lane;
+  const int64_t m = blockIdx.x, xb = m * D;
+  const bool in = i < D;
+  const float4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  float4 xv = zero, w4 = zero;
+  if (mode == 0) {
+    xv = load4<true>(X + xb, i, D);
+    w4 = load4<true>(W + woff, i, D);
+  }
+  float t[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int64_t j = 0; j < nsrc; j += 4) {   // four at a time; past the last: the last again, not added
+    float4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = load4<true>(T + (j + u < nsrc ? j + u : nsrc - 1) * ldp + xb, i, D);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) t[c] = j + u < nsrc ? t[c] + at(v[u], c) : t[c];
+  }
+  auto total = [&](const float (*q)[kChunk]) {
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < kNaWaves; ++k) {
+      const float4 v = *(const float4*)(q[k] + 4 * lane);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s[c] = s[c] + at(v, c);
+    }
+    return tree256(s);
+  };
+  *(float4*)(sq[0][wv] + 4 * lane) = float4{t[0] * t[0], t[1] * t[1], t[2] * t[2], t[3] * t[3]};
+  __syncthreads();
+  const float rs = rsqrt_exact(total(sq[0]) / (float)D + eps);
+  float y[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) y[c] = mode == 0 ? (at(xv, c) + t[c] * rs * at(w4, c)) * scale : t[c];
+  if (in) *(float4*)(X + xb + i) = float4{y[0], y[1], y[2], y[3]};
+  *(float4*)(sq[1][wv] + 4 * lane) = in ? float4{y[0] * y[0], y[1] * y[1], y[2] * y[2], y[3] * y[3]} : zero;
+  __syncthreads();
+  if (wv != 0) return;
+  const float r2 = total(sq[1]);
+  if (lane == 0) ST[stoff + m] = rsqrt_exact(r2 / (float)D + eps);
+}
+
 // engine/llm/lops.js:418-433, engine/llm/lops_spec.js:329-343: (value, index) with ties to the lower index. A running
 // best is never NaN, so "better" is a total order on what is combined: any order of the reduction gives its result. One
 // workgroup of 16 waves per row, four pairs in flight per thread (the 4096 tile maxima of a 262144-row head in one
@@ -327,6 +380,12 @@ extern "C" int p0_normadd(const p0_normadd_args_t* a) {
   if (building_chain())
     return chain_add_normadd(a->t, nsrc, ldp, a->w, a->w_off, a->x, a->st, a->st_off, D, M, eps, a->scale, (int)a->mode);
   const bool vec = vec_ok(a->t, ldp, D) && vec_ok(a->x, 0, 0) && (a->mode == 1 || vec_ok(a->w, a->w_off, 0));
+  if (vec && D <= kNaWaves * kChunk && M <= 256) {
+    hipLaunchKernelGGL(normadd_few_kernel, dim3((unsigned)M), dim3(kNaThreads), 0, ctx().cur, a->t, nsrc, ldp, a->w, a->w_off,
+                       a->x, a->st, a->st_off, (int)D, eps, a->scale, (int)a->mode);
+    P0_LAUNCHED("normadd");
+    return P0_OK;
+  }
   auto k = !vec ? normadd_kernel<false, 4, false> : D <= 8 * kChunk ? normadd_kernel<true, 8, true> : normadd_kernel<true, 8, false>;
   hipLaunchKernelGGL(k, dim3((unsigned)M), dim3(64), 0, ctx().cur, a->t, nsrc, ldp, a->w,
                      a->w_off, a->x, a->st, a->st_off, D, eps, a->scale, (int)a->mode);

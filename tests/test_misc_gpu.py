@@ -109,9 +109,11 @@ def test_rowstats_aligned_rows_bit_exact(dev, rows, cols, mode):
 
 
 @pytest.mark.parametrize("mode", [0, 1])
-@pytest.mark.parametrize("D,M,nsrc", [(4, 1, 1), (1000, 3, 5), (2048, 2, 8), (2052, 2, 4), (6148, 1, 3)])
+@pytest.mark.parametrize("D,M,nsrc", [(4, 1, 1), (1000, 3, 5), (2048, 2, 8), (2052, 2, 4), (6148, 1, 3), (100, 256, 3),
+                                      (100, 257, 3)])
 def test_normadd_aligned_rows_bit_exact(dev, D, M, nsrc, mode):
-    """16-byte aligned rows, in registers (up to 2048 values) and in two passes, partials in fours with a remainder"""
+    """16-byte aligned rows, few (up to 256: a workgroup a row) and many, in registers (up to 2048 values) and in two passes,
+    partials in fours with a remainder"""
     t = O.randn(nsrc * M * D, D + nsrc, 0.3).astype(np.float32)
     w = (0.5 + O.rng_uniform(D, D)).astype(np.float32)
     x0 = O.randn(M * D, D + 1).astype(np.float32)
