@@ -522,11 +522,11 @@ static bool plan_wide(std::vector<GemvP>& ops, int G) {
   return true;
 }
 
-// q8g64s.t64 at M = 1 in splits of more than 2048 k (smaller ones: gemv1.hip): one workgroup per (64-row tile, split),
-// gemv_q8.hip
+// q8g64s.t64 at M = 1 where gemv1.hip does not take it: one workgroup per (64-row tile, split), gemv_q8.hip
 static int launch_q8(GemvP& p, const char* op) {
-  // q8_gemv1_kernel: 16 waves per (tile, split), whose LDS holds at most 3072 k
-  if (p.kPer <= 3072) {
+  // q8_gemv1_kernel: 16 waves per (tile, split), for splits of 1024-3072 k (16-48 groups; its LDS holds no more, and a
+  // split of 4 groups ran faster on the 4-wave kernel: 3.9 against 4.9 us)
+  if (p.kPer >= 1024 && p.kPer <= 3072) {
     // K-slices across workgroups (p.nks) when the tiles and splits leave most CUs idle: up to ~192 workgroups, at
     // least 8 groups (512 k) a slice (measured at the E2B 8-bit shapes: 6.2-9.3 us per launch against 6.9-10.9 with
     // one workgroup per split; p0_gemv_tune knob 5 sets the count)

@@ -209,8 +209,20 @@ static void launch_enc(const GemvP& p, hipStream_t s) {
 // Splits of at most 2048 k (a wave's records of more do not fit its registers). A q4 op of more than 1024 tiles streams
 // from HBM on gemv.hip's kernel: 262144 x 2048 61.2 us there and 61.5 here, with a softcap 66.4 and 70.8; at 65536 rows
 // 20.8 and 18.9, 21.8 and 20.3
+//
+// A short split leaves most of a workgroup's 8 waves without records (a wave takes 128 k of a q4 row at a time, 64 of a
+// q8 row), which a call of several items per workgroup, or of a softcap's 4 blocks per item, pays for item by item: such
+// calls stay on gemv.hip's and gemv_q8.hip's kernels. Per recorded launch, us here / there: q4 geglu 16384 x 320 7.8 / 5.2,
+// x 960 9.5 / 8.4, x 1280 10.0 / 10.2, 4096 x 320 (512 blocks) 4.1 / 4.9; q4 store 16384 x 640 5.2 / 5.1, x 960 5.6 / 6.1,
+// 8192 x 320 4.0 / 4.6; q4 softcap 16384 x 640 6.1 / 5.8, x 960 6.7 / 6.8, 1024 x 320 5.4 / 5.0, x 960 5.5 / 6.2;
+// q8 geglu 16384 x 1024 11.3 / 11.0, 4096 x 320 4.8 / 6.3; q8 store 16384 x 320 6.0 / 5.3, x 640 6.6 / 7.3; q8 softcap
+// 4096 x 320 7.3 / 5.8, 16384 x 1024 8.9 / 8.7.
 bool gemv1_takes(const GemvP& p) {
-  return p.kPer <= kGmPass && (p.enc == P0_ENC_Q8G64S_T64 || p.NT <= 1024);
+  const bool q8 = p.enc == P0_ENC_Q8G64S_T64, geglu = p.epi == P0_EPI_GEGLU;
+  if (p.kPer > kGmPass || (!q8 && p.NT > 1024)) return false;
+  if (p.epi == P0_EPI_SOFTCAP) return p.kPer > (q8 ? 1024 : 640);
+  const int64_t blocks = (int64_t)(p.N / 16) * (geglu ? 2 : 1) * p.nsplit;
+  return blocks <= 512 || p.kPer >= (geglu ? (q8 ? 1088 : 1280) : (q8 ? 640 : 960));
 }
 
 void launch_gemv1(const GemvP& p, hipStream_t s) {

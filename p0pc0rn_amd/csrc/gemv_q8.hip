@@ -1,7 +1,7 @@
-// gemv_q8.hip - the q8g64s.t64 GEMV (M = 1, splits of more than 2048 k) on gfx950: the reference's other weight encoding
+// gemv_q8.hip - the q8g64s.t64 GEMV (M = 1, where gemv1.hip does not take it) on gfx950: the reference's other weight encoding
 // on the same call surface
 // (engine/llm/lops.js:74-80), with the same prologues, epilogues and split semantics as the q4 kernels
-// (gemv_kernels.hpp). Splits of at most 2048 k are in gemv1.hip, its GEMV-M (2-16 rows) in gemvm.hip.
+// (gemv_kernels.hpp). Most splits of at most 2048 k are in gemv1.hip (gemv1_takes), its GEMV-M (2-16 rows) in gemvm.hip.
 //
 // Data layout (packQ8, engine/kcheck.js:39-52): a weight W[N][K] is a sequence of 4224-byte records, record (tile, g)
 // = rows 64 tile .. + 63, k = 64 g .. + 63, tile-major. Bytes [64 r, 64 r + 64) are row r's 64 signed codes in k order;

@@ -326,6 +326,11 @@ def test_gemvM_matrix_core_shapes(dev, M, N, K, pro, epi, kPer):
          gemvM=True).check(f"gemvM M={M} {N}x{K} {pro} {epi}")
 
 
+def one_row(N, K, pro, epi, kPer):
+    Case(1, N, K, pro, epi, kPer=kPer, seed=70, w_off=4, rowB=3 if pro in ("raw", "rms") else 0, ldx=K + 5).check(
+        f"gemv {N}x{K} {pro} {epi}")
+
+
 @pytest.mark.parametrize("N,K,pro,epi,kPer", [
     (64, 32, "raw", "store", 0),                # one group: one quarter of one wave has work
     (128, 5 * 32, "rms", "geglu", 0),           # a second wave with one group of its quad
@@ -343,8 +348,17 @@ def test_gemvM_matrix_core_shapes(dev, M, N, K, pro, epi, kPer):
 ])
 def test_gemv_one_row_shapes(dev, N, K, pro, epi, kPer):
     """gemv1.hip where its pieces end, on both sides of its rule (kPer, tiles), x rows and weights at 4-byte alignment"""
-    Case(1, N, K, pro, epi, kPer=kPer, seed=70, w_off=4, rowB=3 if pro in ("raw", "rms") else 0, ldx=K + 5).check(
-        f"gemv {N}x{K} {pro} {epi}")
+    one_row(N, K, pro, epi, kPer)
+
+
+# many items of short splits, on both sides of the rule that keeps them on gemv.hip's kernel
+@pytest.mark.parametrize("N,K,pro,epi,kPer", [
+    (8192, 64, "rms", "store", 0), (8256, 928, "raw", "store", 0), (16448, 960, "rms", "store", 0),
+    (4096, 64, "raw", "geglu", 0), (4160, 1248, "rms", "geglu", 0), (8256, 1280, "pleg", "geglu", 0),
+    (64, 640, "rms", "softcap", 0), (8256, 672, "raw", "softcap", 0), (4160, 1888, "sum", "store", 960),
+])
+def test_gemv_one_row_short_splits(dev, N, K, pro, epi, kPer):
+    one_row(N, K, pro, epi, kPer)
 
 
 @pytest.mark.parametrize("scale", [1e-30, 1e-3, 1e4, 1e30])

@@ -87,6 +87,12 @@ def test_q8_k_slices_across_workgroups(dev, slices, pro, epi, K, kPer):
     (8256, 64, "raw", "softcap", 0),
     (128, 2112, "rms", "geglu", 0),             # splits that gemv_q8.hip takes
     (128, 3072, "raw", "store", 0),
+    (64, 1024, "rms", "softcap", 0),            # short splits, on both sides of the rule that keeps them there
+    (8256, 1088, "rms", "softcap", 0),
+    (4160, 1024, "rms", "geglu", 0),
+    (8256, 1088, "rms", "geglu", 0),
+    (8256, 576, "raw", "store", 0),
+    (16448, 640, "raw", "store", 0),
 ])
 def test_q8_one_row_shapes(dev, N, K, pro, epi, kPer):
     """gemv1.hip's q8 form where its pieces end, and the splits past its rule; the bar of the file's gemvM test"""
