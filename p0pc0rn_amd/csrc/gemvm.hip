@@ -170,6 +170,12 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[c][e] = v[c][e] * rstd * n[e];
         }
+        // what the loads of a chunk past the split returned (other k, other norm weights) is no x' of the row: it must not
+        // set the row's scale
+        if (!in_pass(c, ng)) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[c][e] = 0.0f;
+        }
       }
     }
     // the row's largest |x'| over the wave's k (the lanes of a row are 16 apart): an infinity makes it infinite, a NaN

@@ -373,6 +373,22 @@ def test_gemvM_row_scales(dev, scale):
         _check(yg[m * 128:(m + 1) * 128], yo[m * 128:(m + 1) * 128], f"gemvM row {m}, scale {scale}")
 
 
+@pytest.mark.parametrize("K", [32, 960, 1536, 2560])
+def test_gemvM_row_scale_from_the_split_only(dev, K):
+    """K that leaves waves (or part of one's k) without work: their loads repeat the first group's x beside the last norm
+    weights, which must not count towards the row's scale. The first group's x is 2^30 times the others, damped by its own
+    norm weights: every row keeps the fp32 bar"""
+    c = Case(5, 128, K, "rms", "store", seed=97, gemvM=True)
+    big = np.float32(2.0 ** 30)
+    c.nw[:32] = c.nw[:32] / big
+    for m in range(5):
+        c.x[m * K:m * K + 32] *= big
+        c.stat[c.fields["stat_off"] + 2 * m] = np.float32(0.7 + 0.1 * m)
+    yo, yg = c.run_oracle()[0], c.run_gpu()[0]
+    for m in range(5):
+        _check(yg[m * 128:(m + 1) * 128], yo[m * 128:(m + 1) * 128], f"gemvM row {m}, K {K}")
+
+
 def test_gemvM_infinities_and_nan_keep_to_their_row(dev):
     """rows with an infinity or a NaN are infinite or NaN where the oracle's are, and leave the other rows alone"""
     M, N, K = 5, 128, 2048
