@@ -442,7 +442,7 @@ static int slices(const GemmP& p, int64_t tiles, int steps) {
 static int64_t tiles_of(const GemmP& p, int bm, int bn) { return ((int64_t)p.N + bn - 1) / bn * (((int64_t)p.M + bm - 1) / bm); }
 
 // Forms: whole 64-row weight tiles (the first weight rows multiples of 64), records 16-byte aligned, X' rows and the weight
-// within 32-bit offsets. Then by time: a step of 64 k takes this kernel 1.0 us a round of 256 workgroups and about 4 us a
+// within 32-bit offsets (unsigned ones: rows that go down in memory stay on gemm.hip, which adds 64-bit offsets). Then by time: a step of 64 k takes this kernel 1.0 us a round of 256 workgroups and about 4 us a
 // call, 12 with K slices (the partials); the 256 x 256 tiles of gemm.hip 1.4 us while one round holds them all, and 9 us.
 // Measured (us, this kernel / gemm.hip): M = 256: 3072 x 2048 21 / 55, 16384 x 2048 swiglu 36 / 62, 2048 x 8192 33 / 179;
 // M = 512: 3072 x 3072 35 / 77, 3072 x 9216 75 / 205, 9216 x 3072 95 / 82; M = 1024: 3072 x 9216 128 / 210; M = 2048:
@@ -450,7 +450,7 @@ static int64_t tiles_of(const GemmP& p, int bm, int bn) { return ((int64_t)p.N +
 bool n128_takes(const GemmP& p) {
   const bool sw = p.epi == P0_GEPI_SWIGLU;
   if (p.wr0 % 64 || (sw && p.wr1 % 64) || ((uintptr_t)p.w & 15)) return false;
-  if (p.ldx >= (1 << 21) || (p.Nw >> 6) * p.wG * 1280 >= (1ll << 31)) return false;
+  if (p.ldx < 0 || p.ldx >= (1 << 21) || (p.Nw >> 6) * p.wG * 1280 >= (1ll << 31)) return false;
   const int steps = (p.K + 63) / 64;
   const int64_t small = tiles_of(p, Tile::BMt, Tile::BNt), big = tiles_of(p, 256, 256);
   const int nks = slices(p, small, steps);

@@ -287,3 +287,18 @@ def test_gemm_small_tiles_against_large(dev, M, N, K, wr0, wk0, epi):
     check(small, large, f"gemm small against large tiles {epi}", 2e-6 if f32 else 1e-3)
     untouched = want == init.astype(dt)
     assert np.array_equal(small[untouched], want[untouched])
+
+
+@pytest.mark.parametrize("M,mode", [(40, "f16"), (300, "f16"), (40, "bf16")])
+def test_gemm_rows_going_down_in_memory(dev, M, mode):
+    """a negative x_ld walks the rows of X from the last in memory to the first: 64-bit offsets, so gemm.hip's (the 32-bit
+    buffer offsets of gemm_n128.hip reach upwards only), or the staging's, whose X' rows go up again"""
+    N, K, ld = 128, 288, 296
+    w = _weights(N, K, 31)
+    xf = O.randn(M * ld, 32)
+    x = xf.astype(np.float16) if mode == "f16" else (xf.view(np.uint32) >> 16).astype(np.uint16)
+    f = dict(w_rows=N, w_cols=K, M=M, N=N, K=K, x_mode=capi.XMODE[mode], epi=capi.GEPI["f32"])
+    want, got = run(dict(f, x_ld=-ld, x_off=(M - 1) * ld * 2), dict(w=w, x=x), np.float32, M * N)
+    check(got, want, f"gemm {mode} rows down {M}x{N}x{K}", 1e-5)
+    up, _ = run(dict(f, x_ld=ld), dict(w=w, x=np.ascontiguousarray(x.reshape(M, ld)[::-1])), np.float32, M * N)
+    assert np.array_equal(up.view(np.uint32), want.view(np.uint32))
