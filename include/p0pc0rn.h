@@ -200,7 +200,9 @@ int p0_q4_gemm(const p0_gemm_args_t* a, double* flops_out);
  * static device scratch of 32 MiB (M * K * 2 bytes at most, else P0_EINVAL), allocated with the library's code on each
  * GPU and held until the process ends. Every call on one GPU shares that scratch: calls that may overlap on one GPU
  * (two streams, two threads) race and must be ordered by the caller. Nothing in it needs to start at zero (each call
- * writes all it reads). */
+ * writes all it reads). Both entry points run small calls in K slices whose partial sums meet in the context's split-K
+ * workspace (allocated by p0_open), counted on arrival counters that only GEMMs use and that every call leaves at zero:
+ * a chain whose wait gave up does not disturb a GEMM, but a GEMM, too, must not overlap another op of the context. */
 int p0_q4_gemm_noalloc(const p0_gemm_args_t* a, double* flops_out);
 
 /* ---- bit-exact dequant of whole q4g32a.t64 weights --------------------------------------------------------------- */

@@ -32,6 +32,9 @@ struct Ctx {
   size_t part_floats = 0;
   unsigned* counters = nullptr;
   size_t n_counters = 0;
+  // the GEMM's own, one per tile of a call with K slices: a chain whose wait gave up leaves counts behind in `counters`
+  // until p0_chain_status clears them, and a GEMM enqueued in between must not take them for its own
+  unsigned* gemm_counters = nullptr;
   // fp16 staging of GEMM activations that the MFMA kernel cannot stream as they are (bf16, the f32 prologues,
   // misaligned fp16): grown on demand, never inside a stream capture (ensure_xstage)
   void* xstage = nullptr;

@@ -466,7 +466,7 @@ void launch_n128(const GemmP& p, hipStream_t s) {
   a.spk = (steps + slices(p, tiles, steps) - 1) / slices(p, tiles, steps);
   a.nks = (steps + a.spk - 1) / a.spk;
   a.part = ctx().part;
-  a.cnt = ctx().counters;   // one per tile where there are slices: at most 128 tiles
+  a.cnt = ctx().gemm_counters;   // one per tile where there are slices: at most 128 tiles
   hipLaunchKernelGGL(tile_kernel, dim3((unsigned)(tiles * a.nks)), dim3(Tile::Threads), Tile::Lds, s, a);
 }
 

@@ -82,13 +82,13 @@ __global__ void copy4_kernel(const uint32_t* __restrict__ src, uint32_t* __restr
 
 using namespace p0;
 
-// Split-K workspace: 64 MiB of partial sums and 1 Mi arrival counters per device, in uncached device memory. The
+// Split-K workspace: 64 MiB of partial sums, 1 Mi arrival counters and the GEMM's 256 per device, in uncached device memory. The
 // partials then reach memory when their stores are acknowledged and are read from memory, so the arrival protocol
 // needs no L2 write-back or invalidate (a device-scope fence costs a write-back of the XCD's whole L2). Uncached memory
 // that a kernel has read is never freed while the process runs (allocations made after such a free have been seen
 // holding wrong values), so each device's workspace is allocated once and kept across p0_close / p0_open.
 static constexpr size_t kPartBytes = 64ull << 20;
-static constexpr size_t kCounters = 1ull << 20;
+static constexpr size_t kCounters = 1ull << 20, kGemmCounters = 256, kAllCounters = kCounters + kGemmCounters;
 static constexpr int kWsDevices = 64;
 static float* g_ws_part[kWsDevices] = {};
 static unsigned* g_ws_cnt[kWsDevices] = {};
@@ -128,16 +128,17 @@ int p0_open(int device) {
     P0_HIP(hipExtMallocWithFlags((void**)&g_ws_part[device], kPartBytes, hipDeviceMallocUncached), "p0_open: workspace");
   }
   if (!g_ws_cnt[device]) {
-    P0_HIP(hipExtMallocWithFlags((void**)&g_ws_cnt[device], kCounters * sizeof(unsigned), hipDeviceMallocUncached),
+    P0_HIP(hipExtMallocWithFlags((void**)&g_ws_cnt[device], kAllCounters * sizeof(unsigned), hipDeviceMallocUncached),
            "p0_open: workspace");
   }
   c.part = g_ws_part[device];
   c.counters = g_ws_cnt[device];
-  P0_HIP(hipMemset(c.counters, 0, kCounters * sizeof(unsigned)), "p0_open: workspace");
+  P0_HIP(hipMemset(c.counters, 0, kAllCounters * sizeof(unsigned)), "p0_open: workspace");
   P0_HIP(hipDeviceSynchronize(), "p0_open");
   if (int r = gemm_init()) return r;
   c.part_floats = kPartBytes / sizeof(float);
   c.n_counters = kCounters;
+  c.gemm_counters = c.counters + kCounters;
   c.cur = c.own;
   c.cu_count = c.prop.multiProcessorCount;
   c.device = device;
@@ -167,7 +168,7 @@ int p0_device_info(p0_device_info_t* out) {
   out->hbm_bytes = (int64_t)c.prop.totalGlobalMem;
   out->lds_bytes_per_cu = (int64_t)c.prop.maxSharedMemoryPerMultiProcessor;
   out->clock_khz = c.prop.clockRate;
-  out->workspace_bytes = (int64_t)(kPartBytes + kCounters * sizeof(unsigned));
+  out->workspace_bytes = (int64_t)(kPartBytes + kAllCounters * sizeof(unsigned));
   return P0_OK;
 }
 

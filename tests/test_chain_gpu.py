@@ -769,3 +769,49 @@ def test_chain_small_and_ragged_shapes(dev, enc):
     ch.free()
     for b in dw + ys + [x, mx]:
         b.free()
+
+
+def test_gemm_after_a_chain_that_gave_up(dev):
+    """a GEMM cut into K slices, enqueued between a chain whose waits gave up part of the way (a tiny poll limit) and the
+    p0_chain_status that clears what it left: the GEMM counts its slices on counters of its own, so its result is the
+    usual one bit for bit. The chain runs on the general kernel, its ops in many K slices"""
+    N, K, ops = 512, 2048, 6
+    M2, N2, K2 = 200, 256, 2048      # 4 tiles of 128 x 128, 4 slices each
+    w, w2 = capi.to_device(_w(N, K, 41)), capi.to_device(_w(N2, K2, 42))
+    x = capi.to_device(O.randn(K, 43))
+    y = [capi.Buffer(2048 * 4).fill_u32(0) for _ in range(ops)]
+    xh = [capi.to_device(O.randn(M2 * K2, 44 + i).astype(np.float16)) for i in range(2)]   # taken in turn: partials differ
+    z = capi.Buffer(M2 * N2 * 4)
+
+    def enqueue():
+        for i in range(ops):
+            capi.q4_gemv(capi.gemv_args(w=w, w_rows=N, w_cols=K, x=y[i - 1] if i else x, N=N, K=K, y=y[i]))
+
+    def gemm(i):
+        z.fill_u32(NAN)
+        capi.q4_gemm(capi.gemm_args(w=w2, w_rows=N2, w_cols=K2, x=xh[i], M=M2, N=N2, K=K2, epi=capi.GEPI["f32"], y=z))
+
+    old = [(k, capi.chain_tune(k, v)) for k, v in ((1, 1), (4, 0))]
+    spin = capi.chain_tune(2, -1)
+    try:
+        ch = capi.chain(enqueue)
+        want = []
+        for i in range(2):
+            gemm(i)
+            want.append(z.read(np.uint32))
+        gave_up = 0
+        for n, limit in enumerate((1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 17, 20, 25, 30, 40, 50) * 8):
+            capi.chain_tune(2, limit)
+            ch.run()
+            gemm(n % 2)
+            got = z.read(np.uint32)
+            gave_up += ch.status()
+            assert np.array_equal(got, want[n % 2]), f"poll limit {limit}"
+        print("runs that gave up:", gave_up, flush=True)
+        ch.free()
+    finally:
+        capi.chain_tune(2, spin)
+        for k, v in old:
+            capi.chain_tune(k, v)
+    for b in [w, w2, x, z] + xh + y:
+        b.free()
