@@ -522,11 +522,12 @@ static bool plan_wide(std::vector<GemvP>& ops, int G) {
   return true;
 }
 
-// q8g64s.t64 at M = 1 where gemv1.hip does not take it: one workgroup per (64-row tile, split), gemv_q8.hip
-static int launch_q8(GemvP& p, const char* op) {
+// q8g64s.t64 at M = 1 where gemv1.hip does not take it, and at M > 1 below g_mf_min_m: one workgroup per (64-row tile,
+// split, x row), gemv_q8.hip
+static int launch_q8(GemvP& p, int M, const char* op) {
   // q8_gemv1_kernel: 16 waves per (tile, split), for splits of 1024-3072 k (16-48 groups; its LDS holds no more, and a
   // split of 4 groups ran faster on the 4-wave kernel: 3.9 against 4.9 us)
-  if (p.kPer >= 1024 && p.kPer <= 3072) {
+  if (M == 1 && p.kPer >= 1024 && p.kPer <= 3072) {
     // K-slices across workgroups (p.nks) when the tiles and splits leave most CUs idle: up to ~192 workgroups, at
     // least 8 groups (512 k) a slice (measured at the E2B 8-bit shapes: 6.2-9.3 us per launch against 6.9-10.9 with
     // one workgroup per split; p0_gemv_tune knob 5 sets the count)
@@ -549,14 +550,15 @@ static int launch_q8(GemvP& p, const char* op) {
     P0_LAUNCHED(op);
     return P0_OK;
   }
-  hipLaunchKernelGGL(q8_kernel(), dim3((unsigned)p.NT, (unsigned)p.nsplit), dim3(256), q8_lds_bytes(), ctx().cur, p);
+  hipLaunchKernelGGL(q8_kernel(), dim3((unsigned)p.NT, (unsigned)p.nsplit, (unsigned)M), dim3(256), q8_lds_bytes(),
+                     ctx().cur, p);
   P0_LAUNCHED(op);
   return P0_OK;
 }
 
 static int launch(GemvP& p, int M, const char* op) {
   ChainBuild* cb = g_chain;
-  if (!cb && M >= 2 && (p.enc == P0_ENC_Q8G64S_T64 || M >= g_mf_min_m)) {   // the matrix-core GEMV-M
+  if (!cb && M >= 2 && M >= g_mf_min_m) {   // the matrix-core GEMV-M
     launch_gemvm(p, ctx().cur);
     P0_LAUNCHED(op);
     return P0_OK;
@@ -566,7 +568,7 @@ static int launch(GemvP& p, int M, const char* op) {
     P0_LAUNCHED(op);
     return P0_OK;
   }
-  if (p.enc == P0_ENC_Q8G64S_T64 && !cb) return launch_q8(p, op);
+  if (p.enc == P0_ENC_Q8G64S_T64 && !cb) return launch_q8(p, M, op);
   if (cb && cb->M == 0) {   // the chain's first GEMV fixes M and the workgroup shape
     cb->M = M;
     cb->W = M == 1 ? g_chain_waves : 8;

@@ -1,7 +1,8 @@
-// gemv_q8.hip - the q8g64s.t64 GEMV (M = 1, where gemv1.hip does not take it) on gfx950: the reference's other weight encoding
-// on the same call surface
-// (engine/llm/lops.js:74-80), with the same prologues, epilogues and split semantics as the q4 kernels
-// (gemv_kernels.hpp). Most splits of at most 2048 k are in gemv1.hip (gemv1_takes), its GEMV-M (2-16 rows) in gemvm.hip.
+// gemv_q8.hip - the q8g64s.t64 GEMV (M = 1, where gemv1.hip does not take it) on gfx950: the reference's other weight
+// encoding on the same call surface (engine/llm/lops.js:74-80), with the same prologues, epilogues and split semantics as
+// the q4 kernels (gemv_kernels.hpp). Most splits of at most 2048 k are in gemv1.hip (gemv1_takes), its GEMV-M (2-16 rows)
+// in gemvm.hip; a caller who keeps GEMV-M calls off the matrix cores (p0_gemv_tune knob 4) gets them here in fp32, an x row
+// per workgroup.
 //
 // Data layout (packQ8, engine/kcheck.js:39-52): a weight W[N][K] is a sequence of 4224-byte records, record (tile, g)
 // = rows 64 tile .. + 63, k = 64 g .. + 63, tile-major. Bytes [64 r, 64 r + 64) are row r's 64 signed codes in k order;
@@ -33,7 +34,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const bool pair = p.epi == P0_EPI_GEGLU;
   const int T = pair ? 2 : 1;
-  const int tile0 = blockIdx.x, split = blockIdx.y;
+  const int tile0 = blockIdx.x, split = blockIdx.y, m = blockIdx.z;   // m: the x row
   const int64_t tiles[2] = {tile0, tile0 + (pair ? p.NT : 0)};
   const int k0s = split * p.kPer, k1s = min(p.K, k0s + p.kPer);
 
@@ -41,7 +42,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
   for (int c0 = k0s; c0 < k1s; c0 += kQ8Chunk) {
     const int c1 = min(k1s, c0 + kQ8Chunk), ng = (c1 - c0) >> 6;
     __syncthreads();   // the previous chunk's x' is no longer read
-    for (int i = tid; i < kQ8Chunk; i += kQ8Threads) xs[i] = c0 + i < c1 ? prologue<false>(p, 0, c0 + i) : 0.0f;
+    for (int i = tid; i < kQ8Chunk; i += kQ8Threads) xs[i] = c0 + i < c1 ? prologue<false>(p, m, c0 + i) : 0.0f;
     __syncthreads();
     if (tid < kQ8CG) {   // group sums in k order
       float s = 0.0f;
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_gemv_kernel(GemvP p) {
     for (int w = 1; w < kQ8Waves; ++w) v += red[(w * 2 + t) * 64 + lane];
     tot[t] = v;
   }
-  epilogue<false>(p, split, 0, tile0, lane, tot[0], tot[1]);
+  epilogue<false>(p, split, m, tile0, lane, tot[0], tot[1]);
 }
 
 // M = 1 (gemv, the decode case): a workgroup of 16 waves per (64-row tile, split), every wave's record loads issued

@@ -335,10 +335,41 @@ def test_q8_ops_join_only_pipelined_chains(dev):
         v.free()
 
 
+@pytest.fixture(params=["valu", "mfma"])
+def mf(request):
+    """p0_gemv_tune knob 4: GEMV-M calls on the fp32 VALU kernel (17) or on the matrix cores (2, the default)"""
+    old = capi.gemv_tune(4, 2 if request.param == "mfma" else 17)
+    yield request.param
+    capi.gemv_tune(4, old)
+
+
+def test_q8_gemvM_valu_keeps_fp32(dev):
+    """knob 4 = 17 keeps a q8 GEMV-M off the matrix cores: x' stays fp32 whatever else its row holds. One x of 2^40 meets
+    only zero weights; under one scale per row the others' bits would be lost beside it"""
+    M, N, K = 3, 128, 320
+    w = np.asarray(_q8(N, K, 81)).view(np.uint8).reshape(N // 64, K // 64, 4224).copy()
+    w[:, 0, 4096:] = 0   # the first group's scales
+    x = O.randn(M * K, 82)
+    x[0::K] = 2.0 ** 40
+    f = dict(w_enc=2, w_rows=N, w_cols=K, M=M, N=N, K=K)
+    want = np.full(M * N, np.nan, np.float32)
+    O.q4_gemvM(capi.gemvm_args(**f, w=w.ctypes.data, x=x.ctypes.data, y=want.ctypes.data))
+    wb, xb, yb = capi.to_device(w), capi.to_device(x), capi.Buffer(want.nbytes).fill_u32(0x7FC00000)
+    old = capi.gemv_tune(4, 17)
+    try:
+        capi.q4_gemvM(capi.gemvm_args(**f, w=wb, x=xb, y=yb))
+    finally:
+        capi.gemv_tune(4, old)
+    got = yb.read(np.float32)
+    assert np.all(np.isfinite(got)) and rel_l2(got, want) <= 2e-5
+    for v in (wb, xb, yb):
+        v.free()
+
+
 @pytest.mark.parametrize("M,N,K,kPer,epi", [(2, 64, 64, 0, "store"), (16, 192, 9 * 64, 0, "geglu"), (5, 128, 2112, 0, "geglu"),
                                             (7, 320, 4160, 2048, "store"), (5, 4160, 128, 0, "store"),
                                             (3, 16448, 64, 0, "store")])
-def test_q8_gemvM_shapes(dev, M, N, K, kPer, epi):
+def test_q8_gemvM_shapes(dev, mf, M, N, K, kPer, epi):
     """the q8 GEMV-M where its pieces end (one group, one past eight, a second pass of one group, kPer splits, items of 1,
     2 and 4 blocks, several items a workgroup), rms prologue, x and weights at 4-byte alignment, rows of y apart"""
     rows, ldx, ldm, ns = (2 * N if epi == "geglu" else N), K + 3, N + 5, (-(-K // kPer) if kPer else 1)
