@@ -106,9 +106,20 @@ __device__ __forceinline__ AuxP aux_fields(const GemvP* pp) {
 
 // normadd (engine/llm/lops.js:153-170) of rows of up to 2048 values over up to 4 partials, every normadd of a decode
 // layer: the partials, the residual and the norm weights are all in flight before the first is used, one memory round
-// trip instead of one per partial and pass. A function of its own, so that it saves few registers of its caller's. With
-// this and the scalar fields the two normadds of a layer cost a chained M = 1 token (30 layers) 6 us each, the flags before and after them included; 16 before.
+// trip instead of one per partial and pass. With this and the scalar fields the two normadds of a layer cost a chained
+// M = 1 token (30 layers) 6 us each, the flags before and after them included; 16 before.
+// A function of its own beside aux_run, and few registers: what the chain kernels hold across the two calls lives in the
+// registers that neither callee uses, and what does not fit is spilled by every chain, also one without a normadd. With
+// 64-bit addresses per load this took 134 VGPRs (chains of 5 rows without normadds 337 -> 389 us over 8 layers, M = 3 281
+// -> 306, M = 2 222 -> 235); buffer loads, one resource per row and one offset for all, take 115 and the kernels spill as
+// little as with aux_run alone (tests/test_build_resources.py holds them to it).
 __host__ __device__ inline bool aux_normadd_fits(int64_t D, int64_t n) { return D <= kAuxBatch * 256 && n <= 4; }
+// elements tc + 256 u of the D at a (uniform), 0 past them (the resource ends there); sc1: device-coherent, as aux_ldf
+__device__ __forceinline__ void aux_row(const float* a, int D, int tc, float (&v)[kAuxBatch]) {
+  const auto r = __builtin_amdgcn_make_buffer_rsrc((void*)a, 0, D * 4, 0x00020000);
+#pragma unroll
+  for (int u = 0; u < kAuxBatch; ++u) v[u] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, tc * 4, u * 1024, 16));
+}
 __device__ __noinline__ unsigned aux_normadd(const GemvP* pp, int b, int G, int tc, lds_f32* lds, lds_u32* ctr, unsigned gen) {
 #pragma clang fp contract(off)
   const AuxP p = aux_fields(pp);
@@ -124,17 +135,11 @@ __device__ __noinline__ unsigned aux_normadd(const GemvP* pp, int b, int G, int 
       float v[4][kAuxBatch];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
-        if (j < p.an)
-#pragma unroll
-          for (int u = 0; u < kAuxBatch; ++u)
-            v[j][u] = tc + u * 256 < D ? aux_ldf(p.asrc + j * p.aldp + xb + tc + u * 256) : 0.0f;
-      if (p.amode == 0)
-#pragma unroll
-        for (int u = 0; u < kAuxBatch; ++u) {
-          const bool in = tc + u * 256 < D;
-          xv[u] = in ? aux_ldf(p.adst + xb + tc + u * 256) : 0.0f;
-          wv8[u] = in ? aux_ldf(p.aw + p.awOff + tc + u * 256) : 0.0f;
-        }
+        if (j < p.an) aux_row(p.asrc + j * p.aldp + xb, D, tc, v[j]);
+      if (p.amode == 0) {
+        aux_row(p.adst + xb, D, tc, xv);
+        aux_row(p.aw + p.awOff, D, tc, wv8);
+      }
 #pragma unroll
       for (int u = 0; u < kAuxBatch; ++u) {
         t[u] = 0.0f;
