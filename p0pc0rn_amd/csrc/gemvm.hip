@@ -18,6 +18,10 @@
 //    term's sums of x' come from two MFMAs per group against a constant operand, already in the result layout.
 //  * A workgroup with more items than one (a head's 262144 rows) loads the next item's records before it reduces this
 //    one's, and keeps x'.
+//  * A split of more than 2048 k is taken 2048 at a time; where its items leave CUs idle, those passes are slices of K
+//    over workgroups, whose sums meet in the split-K workspace (the GEMV's protocol). 5 rows, one split: 64 x 8192
+//    11.3 -> 7.0 us, 512 x 16384 17.0 -> 8.6, geglu 512 x 8192 17.9 -> 9.9 (before: the kernel that cut K over
+//    workgroups for every call; without slices 14.5, 27.2 and 22.5).
 // Bound: at the E2B shapes, one launch's chain (arguments, x, the split of x', the records, the reduction, the stores);
 // for a head, HBM. Per launch, recorded over weights in HBM, 5 rows: q4 gate_up 2 x 8192 x 2048 11.1 us (18.4 before: x'
 // staged in LDS by every workgroup, K split over two workgroups with partials in uncached memory), 3072 x 2048 6.7 (11.0),
@@ -45,8 +49,9 @@ __device__ __forceinline__ half8_t codes_q8(uint32_t w0, uint32_t w1) {
   return __builtin_bit_cast(half8_t, u);
 }
 
-// One launch: grid (workgroups, splits); workgroup pos takes items [pos ipw, (pos + 1) ipw) of its split
-template <int ENC, int NBK, bool GEGLU, bool PLEG>
+// One launch: grid (workgroups, splits x K slices); workgroup pos takes items [pos ipw, (pos + 1) ipw) of its split. SLICED:
+// p.nks > 1 slices of a split, one item per workgroup
+template <int ENC, int NBK, bool GEGLU, bool PLEG, bool SLICED>
 __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   constexpr bool Q4 = ENC == P0_ENC_Q4G32A_T64;
   constexpr int GK = Q4 ? 32 : 64;             // k per group
@@ -56,11 +61,14 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   __shared__ __attribute__((aligned(16))) float nws[kGmWaves][256];   // the waves' norm weights (rms), in k order
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int M = p.M, l16 = lane & 15, q = lane >> 4, m = min(l16, M - 1);
-  const int pos = stage_pos(blockIdx.x, p.wgs), split = blockIdx.y;
+  const int pos = stage_pos(blockIdx.x, p.wgs);
+  const int split = SLICED ? (int)blockIdx.y / p.nks : blockIdx.y, ks = SLICED ? (int)blockIdx.y - split * p.nks : 0;
   const int it0 = pos * p.ipw, it1 = min(p.items, it0 + p.ipw);
   if (it0 >= it1) return;
-  const int k0s = split * p.kPer, k1s = min(p.K, k0s + p.kPer);
-  const int passes = (k1s - k0s + kGmPass - 1) / kGmPass;
+  // the workgroup's k: its split, or its slice of it (none, for the last slices of a last split shorter than the others)
+  const int k0s = split * p.kPer + ks * p.pps * kGmPass;
+  const int k1s = SLICED ? min(min(p.K, (split + 1) * p.kPer), k0s + p.pps * kGmPass) : min(p.K, k0s + p.kPer);
+  const int passes = SLICED ? max(0, (k1s - k0s + kGmPass - 1) / kGmPass) : (k1s - k0s + kGmPass - 1) / kGmPass;
 
   // weight row of block b of item it (a geglu's blocks U .. NBK - 1: the up rows)
   auto block_row = [&](int it, int b) { return (it * U + (GEGLU ? b % U : b)) * 16 + (GEGLU && b >= U ? p.N : 0); };
@@ -286,6 +294,14 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
     }
   };
 
+  // where slice s of this workgroup's item keeps the sum of x row mm, row l16 of block b (h = 1: a geglu's up row)
+  auto slice_at = [&](int s, int mm, int b, int h) {
+    return p.part + ((((int64_t)(split * p.items + it0) * p.nks + s) * (GEGLU ? 2 : 1) + h) * M * U + mm * U + b) * 16 + l16;
+  };
+  auto slice_store = [&](int mm, int b, float v0, float v1) {
+    stf<true>(slice_at(ks, mm, b, 0), v0);
+    if (GEGLU) stf<true>(slice_at(ks, mm, b, 1), v1);
+  };
   auto pass_groups = [&](int ps) { return min(k1s - (k0s + ps * kGmPass), kGmPass) / GK; };
   for (int it = it0; it < it1; ++it) {
     float tot[NBK][4];
@@ -323,19 +339,66 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
         for (int w = 0; w < kGmWaves; ++w) v1 += rd[w][NBK - U + b][mm & 3][at];
       }
       const int n = (it * U + b) * 16 + l16;
-      epilogue<false>(p, split, mm, n >> 6, n & 63, v0, v1);
+      if (SLICED) slice_store(mm, b, v0, v1);
+      else epilogue<false>(p, split, mm, n >> 6, n & 63, v0, v1);
     }
   }
+  if constexpr (!SLICED) return;
+  // the last of an item's slices to arrive adds their sums in slice order. The workspace
+  // is uncached memory: a store is in memory once acknowledged, so the arrival count needs no fence
+  __shared__ int s_last;
+  __builtin_amdgcn_s_waitcnt(0);
+  __syncthreads();
+  if (tid == 0) {
+    auto* c = P0_GLOBAL(unsigned, p.cnt + split * p.items + it0);
+    s_last = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(p.nks - 1);
+    if (s_last) __hip_atomic_exchange(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // leave it at zero
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int r = tid >> 4; r < M * U; r += kGmThreads / 16) {
+    const int mm = r / U, b = r - mm * U, n = (it0 * U + b) * 16 + l16;
+    float v[2] = {0.0f, 0.0f};
+    for (int s0 = 0; s0 < p.nks; s0 += 8) {   // 8 slices in flight; past the last: the last again, not added
+      float t[8][GEGLU ? 2 : 1];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+#pragma unroll
+        for (int h = 0; h < (GEGLU ? 2 : 1); ++h) t[u][h] = ldf<true>(slice_at(min(s0 + u, p.nks - 1), mm, b, h));
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (s0 + u < p.nks)
+#pragma unroll
+          for (int h = 0; h < (GEGLU ? 2 : 1); ++h) v[h] += t[u][h];
+    }
+    epilogue<false>(p, split, mm, n >> 6, n & 63, v[0], v[1]);
+  }
+}
+
+// Splits of several passes: a slice of whole passes per workgroup, as many slices as leave every workgroup one item and a CU
+// of its own
+static void slice_plan(const GemvP& p, GmPlan& pl) {
+  GmP& g = pl.args;
+  const int passes = (min(p.kPer, p.K) + kGmPass - 1) / kGmPass, wgs = g.items * p.nsplit;
+  const int most = wgs <= 256 ? 256 / wgs : 1;
+  g.pps = (passes + most - 1) / most;
+  g.nks = (passes + g.pps - 1) / g.pps;
+  g.part = ctx().part;      // at most 256 workgroups' 16 x 64 sums (a geglu's 16 x 32 twice): 1 MiB of its 64
+  g.cnt = ctx().counters;   // nsplit * items <= 256
+  pl.grid.y = (unsigned)(p.nsplit * g.nks);   // gm_plan gives a workgroup more items than one only past 256
 }
 
 template <int ENC>
 static void launch_enc(const GemvP& p, hipStream_t s) {
-  const GmPlan pl = gm_plan(p, 512);
-  const GmP& g = pl.args;
+  GmPlan pl = gm_plan(p, 512);
+  GmP& g = pl.args;
+  slice_plan(p, pl);
   const bool geglu = p.epi == P0_EPI_GEGLU;
   const int nbk = pl.nbk;
-  const bool pleg = p.pro == P0_PRO_PLEG;
-#define P0_GM(NBK, GEGLU) (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true> : gemvm_kernel<ENC, NBK, GEGLU, false>)
+  const bool pleg = p.pro == P0_PRO_PLEG, sliced = g.nks > 1;
+#define P0_GM(NBK, GEGLU)                                                                                               \
+  (sliced ? (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true, true> : gemvm_kernel<ENC, NBK, GEGLU, false, true>)             \
+          : (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true, false> : gemvm_kernel<ENC, NBK, GEGLU, false, false>))
   auto k = geglu ? (nbk == 4 ? P0_GM(4, true) : P0_GM(2, true))
                  : nbk == 4 ? P0_GM(4, false) : nbk == 2 ? P0_GM(2, false) : P0_GM(1, false);
 #undef P0_GM

@@ -326,6 +326,27 @@ def test_gemvM_matrix_core_shapes(dev, M, N, K, pro, epi, kPer):
          gemvM=True).check(f"gemvM M={M} {N}x{K} {pro} {epi}")
 
 
+@pytest.mark.parametrize("M,N,K,pro,epi", [
+    (2, 64, 2080, "raw", "store"),              # a second slice of one group
+    (5, 128, 16384, "rms", "store"),            # 8 slices of one pass
+    (3, 64, 32768, "raw", "store"),             # 16 slices: two rounds of the last workgroup's loads
+    (16, 1024, 6176, "raw", "store"),           # 64 items, the last slice of one group
+    (7, 512, 16416, "raw", "geglu"),            # 32 items of a gate and an up block, slices of two passes
+    (4, 320, 8192, "rms", "softcap"),           # whole tiles
+    (2, 2112, 4128, "raw", "store"),            # 132 items: one slice
+    (9, 64, 4096, "pleg", "geglu"),
+])
+def test_gemvM_long_split_in_k_slices(dev, M, N, K, pro, epi):
+    """one split of more than 2048 k: its passes over K in slices over workgroups, where the rows of weights leave CUs
+    idle (each slice's sums through the workspace, added in slice order by the last to arrive): the file's fp32 bar, the
+    same bits again, and counters back at zero (a second call)"""
+    c = Case(M, N, K, pro, epi, seed=60 + M, w_off=4, rowB=3 if pro != "pleg" else 0, ldx=K + 5, ldm=N + 7, gemvM=True)
+    c.check(f"gemvM M={M} {N}x{K} {pro} {epi}, K slices")
+    a, b = c.run_gpu(), c.run_gpu()
+    assert np.array_equal(a[0].view(np.uint32), b[0].view(np.uint32))
+    assert np.array_equal(a[1].view(np.uint32), b[1].view(np.uint32))
+
+
 def one_row(N, K, pro, epi, kPer):
     Case(1, N, K, pro, epi, kPer=kPer, seed=70, w_off=4, rowB=3 if pro in ("raw", "rms") else 0, ldx=K + 5).check(
         f"gemv {N}x{K} {pro} {epi}")

@@ -368,7 +368,8 @@ def test_q8_gemvM_valu_keeps_fp32(dev):
 
 @pytest.mark.parametrize("M,N,K,kPer,epi", [(2, 64, 64, 0, "store"), (16, 192, 9 * 64, 0, "geglu"), (5, 128, 2112, 0, "geglu"),
                                             (7, 320, 4160, 2048, "store"), (5, 4160, 128, 0, "store"),
-                                            (3, 16448, 64, 0, "store")])
+                                            (3, 16448, 64, 0, "store"),
+                                            (6, 128, 6208, 0, "store")])   # K slices over workgroups, the last of one group
 def test_q8_gemvM_shapes(dev, mf, M, N, K, kPer, epi):
     """the q8 GEMV-M where its pieces end (one group, one past eight, a second pass of one group, kPer splits, items of 1,
     2 and 4 blocks, several items a workgroup), rms prologue, x and weights at 4-byte alignment, rows of y apart"""
