@@ -5,8 +5,8 @@
 //
 // Mapping. The weight rows are cut into blocks of 16 (one v_mfma_f32_16x16x32_f16 operand); a workgroup of 8 waves takes
 // an item of NBK blocks (a geglu item: NBK / 2 gate blocks and their up blocks; a softcap item: one 64-row tile) and
-// the whole K range of one kPer split, the waves each an eighth of it, so nothing leaves the workgroup but outputs: no
-// K-slices across workgroups, no partials in memory, one barrier per item (the waves' sums meet in LDS).
+// the whole K range of one kPer split (long splits aside, see below), the waves each an eighth of it, so nothing leaves
+// the workgroup but outputs: no partials in memory, one barrier per item (the waves' sums meet in LDS).
 //  * x' lives in registers. A lane's A operand is 8 consecutive k of one x row: the wave loads its 256 k of every row
 //    straight from x (no LDS), scales each row by a power of two so that its largest |x'| lies in [2^14, 2^15), and
 //    splits it into fp16 hi + lo, so a value within 2^-18 of its row's largest keeps 22 bits, nothing overflows, and
@@ -178,21 +178,16 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) v[c][e] = v[c][e] * rstd * n[e];
         }
-        // what the loads of a chunk past the split returned (other k, other norm weights) is no x' of the row: it must not
-        // set the row's scale
-        if (!in_pass(c, ng)) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[c][e] = 0.0f;
-        }
       }
     }
     // the row's largest |x'| over the wave's k (the lanes of a row are 16 apart): an infinity makes it infinite, a NaN
-    // stays out of it
+    // stays out of it, and so does what the loads of a chunk past the split returned (other k, other norm weights)
     float big = 0.0f;
 #pragma unroll
     for (int c = 0; c < 8; ++c)
+      if (in_pass(c, ng))
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) big = fmaxf(fmaxf(big, __builtin_fabsf(v[c][e])), __builtin_fabsf(v[c][e + 1]));
+        for (int e = 0; e < 8; e += 2) big = fmaxf(fmaxf(big, __builtin_fabsf(v[c][e])), __builtin_fabsf(v[c][e + 1]));
     auto over_row = [](float b) {
       const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(b), __float_as_uint(b), false, false);
       b = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
@@ -205,11 +200,12 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
       big = 0.0f;
 #pragma unroll
       for (int c = 0; c < 8; ++c)
+        if (in_pass(c, ng))
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float a = __builtin_fabsf(v[c][e]);
-          big = fmaxf(big, a < __builtin_inff() ? a : 0.0f);
-        }
+          for (int e = 0; e < 8; ++e) {
+            const float a = __builtin_fabsf(v[c][e]);
+            big = fmaxf(big, a < __builtin_inff() ? a : 0.0f);
+          }
       big = over_row(big);
     }
     const int ex = (int)((__float_as_uint(big) >> 23) & 255u) - 127;   // floor(log2 big); -127 for 0 and subnormals
