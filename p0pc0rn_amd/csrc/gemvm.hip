@@ -58,7 +58,9 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   constexpr int RJ = Q4 ? 2 : 4;               // record loads per block and pass: quads of groups (q4), groups (q8)
   constexpr int U = GEGLU ? NBK / 2 : NBK;     // 16-row blocks of output rows per item
   __shared__ float red[2][kGmWaves][NBK][4][64];
-  __shared__ __attribute__((aligned(16))) float nws[kGmWaves][256];   // the waves' norm weights (rms), in k order
+  // per wave, in the order of its k: the norm weights (rms), or x' of four rows (pleg; kPlegRow apart: fewer bank conflicts)
+  constexpr int kPlegRow = 256 + 32;
+  __shared__ __attribute__((aligned(16))) float nws[kGmWaves][PLEG ? 4 * kPlegRow : 256];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int M = p.M, l16 = lane & 15, q = lane >> 4, m = min(l16, M - 1);
   const int pos = stage_pos(blockIdx.x, p.wgs);
@@ -139,24 +141,74 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   auto finish_x = [&](int kp, int ng) {
     float v[8][8];
     if constexpr (PLEG) {
+      // Two ways to x' = gelu(sum of partials) ev, whose arithmetic is most of a small call. Few rows: the lanes take 4 of the
+      // wave's 256 k each, four rows at a time, and hand x' round through LDS, so that each is worked out once (4 M gelus a
+      // lane). Many rows, or few k: each lane its own operands', chunk by chunk (8 per chunk that the pass holds, 16 / M
+      // times over). The line is where their counts meet, less the first one's round trips: 2048 x 256 (4 chunks), 16 rows
+      // 12.1 us / 7.7, 8 rows 7.9 / 7.5, 3 rows 5.4 / 7.5; 2048 x 2048 (8 chunks), 16 rows 15.3 / 15.1, 8 rows 10.4 / 14.5
+      if (M <= 8 && in_pass(M - 1, ng)) {
+        const int nk = kp + min((wv + kGmWaves * (lane * 4 / RUN)) * RUN + lane * 4 % RUN, ng * GK - 4);
+        for (int r0 = 0; r0 < M; r0 += 4) {
+          u32x4 ev[4];
+          float t[4][4];
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
+          for (int i = 0; i < 4; ++i) {
+            ev[i] = *P0_GLOBAL(const u32x4, p.EV + min(r0 + i, M - 1) * p.evLd + nk);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[c][e] = 0.0f;
-        if (!in_pass(c, ng)) continue;
-        for (int j = 0; j < p.nsrc; ++j) {
-          const float* xr = p.X + j * p.ldp + m * p.ldx + kp + at_k(c, ng) + kq;
-          const u32x4 x0 = *P0_GLOBAL(const u32x4, xr), x1 = *P0_GLOBAL(const u32x4, xr + 4);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            v[c][e] += __uint_as_float(x0[e]);
-            v[c][e + 4] += __uint_as_float(x1[e]);
+            for (int e = 0; e < 4; ++e) t[i][e] = 0.0f;
           }
-        }
-        const float* ev = p.EV + m * p.evLd + kp + at_k(c, ng) + kq;
-        const u32x4 e0 = *P0_GLOBAL(const u32x4, ev), e1 = *P0_GLOBAL(const u32x4, ev + 4);
+          for (int j = 0; j < p.nsrc; ++j) {
+            u32x4 y[4];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[c][e] = gelu_tanh(v[c][e]) * __uint_as_float(e < 4 ? e0[e & 3] : e1[e & 3]);
+            for (int i = 0; i < 4; ++i) y[i] = *P0_GLOBAL(const u32x4, p.X + j * p.ldp + min(r0 + i, M - 1) * p.ldx + nk);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+              for (int e = 0; e < 4; ++e) t[i][e] += __uint_as_float(y[i][e]);
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   // as for nws below
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (r0 + i < M) {
+              float4 f;
+              f.x = gelu_tanh(t[i][0]) * __uint_as_float(ev[i].x);
+              f.y = gelu_tanh(t[i][1]) * __uint_as_float(ev[i].y);
+              f.z = gelu_tanh(t[i][2]) * __uint_as_float(ev[i].z);
+              f.w = gelu_tanh(t[i][3]) * __uint_as_float(ev[i].w);
+              *(float4*)(nws[wv] + i * kPlegRow + lane * 4) = f;
+            }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          if (m >= r0 && m < r0 + 4)
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+              const float* xr = nws[wv] + (m - r0) * kPlegRow + (c / CR) * RUN + kl(c) + kq;
+              const float4 x0 = *(const float4*)xr, x1 = *(const float4*)(xr + 4);
+              v[c][0] = x0.x; v[c][1] = x0.y; v[c][2] = x0.z; v[c][3] = x0.w;
+              v[c][4] = x1.x; v[c][5] = x1.y; v[c][6] = x1.z; v[c][7] = x1.w;
+            }
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[c][e] = 0.0f;
+          if (!in_pass(c, ng)) continue;
+          const int k = kp + at_k(c, ng) + kq;
+          for (int j = 0; j < p.nsrc; ++j) {
+            const float* xr = p.X + j * p.ldp + m * p.ldx + k;
+            const u32x4 x0 = *P0_GLOBAL(const u32x4, xr), x1 = *P0_GLOBAL(const u32x4, xr + 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              v[c][e] += __uint_as_float(x0[e]);
+              v[c][e + 4] += __uint_as_float(x1[e]);
+            }
+          }
+          const float* ev = p.EV + m * p.evLd + k;
+          const u32x4 e0 = *P0_GLOBAL(const u32x4, ev), e1 = *P0_GLOBAL(const u32x4, ev + 4);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[c][e] = gelu_tanh(v[c][e]) * __uint_as_float(e < 4 ? e0[e & 3] : e1[e & 3]);
+        }
       }
     } else {
       if (rms) {

@@ -326,6 +326,15 @@ def test_gemvM_matrix_core_shapes(dev, M, N, K, pro, epi, kPer):
          gemvM=True).check(f"gemvM M={M} {N}x{K} {pro} {epi}")
 
 
+@pytest.mark.parametrize("M,N,K,nsrc,epi", [(2, 64, 32, 1, "store"), (4, 128, 960, 3, "store"), (5, 64, 2048, 2, "geglu"),
+                                            (16, 128, 1184, 1, "store"), (13, 64, 2048, 4, "softcap"), (3, 16448, 288, 2, "store")])
+def test_gemvM_pleg_rows_in_fours(dev, M, N, K, nsrc, epi):
+    """the pleg prologue's x' rows are worked out four at a time: M on both sides of multiples of 4, K that leaves waves
+    or part of one's k without work, several partials"""
+    Case(M, N, K, "pleg", epi, seed=40 + M, w_off=4, ldx=K + 5, ldm=N + 7, gemvM=True, nsrc=nsrc).check(
+        f"gemvM M={M} {N}x{K} pleg of {nsrc} {epi}")
+
+
 @pytest.mark.parametrize("M,N,K,pro,epi", [
     (2, 64, 2080, "raw", "store"),              # a second slice of one group
     (5, 128, 16384, "rms", "store"),            # 8 slices of one pass
