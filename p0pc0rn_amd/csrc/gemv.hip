@@ -42,7 +42,7 @@ static int g_target_waves = 2048;       // waves a call aims for before it split
 static int g_two_tiles_min_nt = 1024;   // output tiles from which a wave streams two tiles
 static int g_min_gpw = 2;               // fewest q4 groups a wave streams when K is split
 static int g_max_kw = 16;               // most waves that share one tile slot's K-slice inside a workgroup
-static int g_mf_min_m = 2;              // fewest x rows a standalone GEMV-M runs on MFMA (17: never)
+static int g_mf_min_m = 2;              // fewest x rows a standalone GEMV-M may run on MFMA (17: never; gemvm_takes)
 static int g_q8_slices = 0;             // q8g64s.t64 GEMV at M = 1: K-slices per split across workgroups (0: planned)
 static int g_pipe_mf_min_m = 3;         // fewest x rows a pipelined chain does its slot arithmetic on MFMA (6: never)
 
@@ -70,7 +70,8 @@ static Plan plan(int M, int NT, int epi, int nsplit, int kPer) {
   const int kws_max = Gs / g_min_gpw > 1 ? Gs / g_min_gpw : 1;
   if (kws > kws_max) kws = kws_max;
   if (kws < 1) kws = 1;
-  const int max_kw = M <= 2 ? g_max_kw : (g_max_kw < 8 ? g_max_kw : 8);   // the kernel's launch bound
+  // the kernel's launch bound (2 rows with 16 waves: 2048 x 8192 13.9 us, with 8 9.6)
+  const int max_kw = M == 1 ? g_max_kw : (g_max_kw < 8 ? g_max_kw : 8);
   pl.kw = kws < max_kw ? kws : max_kw;
   // one tile per slot whose K is split across workgroups anyway: at most 8 waves per slot, so that twice the
   // workgroups (each with half the records to issue and dot) share it
@@ -558,7 +559,7 @@ static int launch_q8(GemvP& p, int M, const char* op) {
 
 static int launch(GemvP& p, int M, const char* op) {
   ChainBuild* cb = g_chain;
-  if (!cb && M >= 2 && M >= g_mf_min_m) {   // the matrix-core GEMV-M
+  if (!cb && M >= 2 && M >= g_mf_min_m && gemvm_takes(p)) {   // the matrix-core GEMV-M
     launch_gemvm(p, ctx().cur);
     P0_LAUNCHED(op);
     return P0_OK;

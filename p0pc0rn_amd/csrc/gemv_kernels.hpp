@@ -560,7 +560,7 @@ __device__ __forceinline__ bool gemv_item(const GemvP& p, int bx, int by, float*
   // largest kw (the workgroup's wave count) with clamped indices, so they issue back to back and wait once; the
   // entries past kw add an exact zero.
   if (p.kw > 1) {
-    constexpr int KWMAX = M <= 2 ? 16 : 8;
+    constexpr int KWMAX = M == 1 ? 16 : 8;
 #pragma unroll
     for (int m = 0; m < M; ++m) {
       __syncthreads();
@@ -804,10 +804,10 @@ __device__ __forceinline__ void staged_op(const GemvP& p, int b, int G, float* s
   }
 }
 
-// One op, one launch: grid (tile blocks, splits x K-slices). Up to 16 waves per workgroup for M <= 2; 8 for larger
+// One op, one launch: grid (tile blocks, splits x K-slices). Up to 16 waves per workgroup for M = 1; 8 for larger
 // M, whose accumulators need the registers (128 VGPRs per lane at 16 waves would spill).
 template <int M, int MODE>
-__global__ __launch_bounds__(M <= 2 ? 1024 : 512) void q4_gemv_kernel(GemvP p) {
+__global__ __launch_bounds__(M == 1 ? 1024 : 512) void q4_gemv_kernel(GemvP p) {
   extern __shared__ __attribute__((aligned(16))) float smem[];   // 16-byte aligned: ds_read_b128 of x
   __shared__ int s_last;
   gemv_item<M, MODE, false>(p, blockIdx.x, blockIdx.y, smem, &s_last, [] { return true; });

@@ -453,6 +453,31 @@ static void launch_enc(const GemvP& p, hipStream_t s) {
   hipLaunchKernelGGL(k, pl.grid, dim3(kGmThreads), 0, s, g);
 }
 
+// q4 calls of few rows that gemv.hip's fp32 kernel (x' staged once a workgroup, K over workgroups) runs faster. The line was
+// taken where both were measured; per recorded launch, us here / there:
+//  * short splits of many blocks leave most of a workgroup's waves without records. 2 rows: 16384 x 256 6.4 / 5.4, x 512 6.6 /
+//    6.1, x 1024 7.4 / 7.4, geglu 16384 x 640 10.6 / 8.7, 2048 x 8192 in splits of 512 8.4 / 7.3, 4096 x 256 (256 blocks) 5.0
+//    / 5.0, 64 x 64 4.6 / 4.0; 3 rows: 16384 x 256 6.5 / 6.1, x 512 6.6 / 6.9, geglu 16384 x 640 10.7 / 10.1; 4 rows: 512 x 8192
+//    in 64 splits 8.2 / 6.8, 16384 x 256 6.5 / 7.0;
+//  * long splits whose passes do not all get a workgroup of their own. 2 rows: 4096 x 8192 16.3 / 12.4, 2048 x 16384 17.6 /
+//    12.7, 2048 x 4096 (one pass each) 7.8 / 8.5, 8192 x 8192 20.3 / 19.4, 8192 x 16384 36.6 / 45.1, geglu 8192 x 4096 17.9 /
+//    16.8; 3 rows: 4096 x 8192 16.7 / 15.8, 2048 x 4096 7.8 / 9.6; a softcap's items of whole tiles: 2 rows 2048 x 2560 11.5 /
+//    9.6, 16384 x 2560 15.2 / 16.3, 3 rows 256 x 2560 10.9 / 9.8.
+bool gemvm_takes(const GemvP& p) {
+  const int M = p.mrows, geglu = p.epi == P0_EPI_GEGLU;
+  if (p.enc == P0_ENC_Q8G64S_T64 || M > 5) return true;
+  const int64_t rows = (int64_t)(p.N / 16) * (geglu ? 2 : 1), blocks = rows * p.nsplit;
+  if (p.kPer > kGmPass) {
+    if (M > 3) return true;
+    if (p.epi == P0_EPI_SOFTCAP) return rows > 256;
+    if (geglu) return M == 3 || rows > 1024;
+    return rows > 256 || blocks * ((p.kPer + kGmPass - 1) / kGmPass) <= 256 || (M == 3 && p.kPer <= 4096);
+  }
+  if (M == 2) return p.kPer > 64 && (p.kPer > 640 || blocks < 512);
+  if (M == 3) return p.kPer > (geglu ? 640 : 256) || blocks < 512;
+  return p.kPer > 256 || p.nsplit < 32;
+}
+
 void launch_gemvm(const GemvP& p, hipStream_t s) {
   if (p.enc == P0_ENC_Q4G32A_T64) launch_enc<P0_ENC_Q4G32A_T64>(p, s);
   else launch_enc<P0_ENC_Q8G64S_T64>(p, s);

@@ -54,6 +54,7 @@ inline GmPlan gm_plan(const GemvP& p, int64_t big) {   // big: blocks from which
   return pl;
 }
 
+bool gemvm_takes(const GemvP& p);                   // do 2..16 rows' op run on gemvm.hip
 void launch_gemvm(const GemvP& p, hipStream_t s);   // p.mrows = 2..16 rows, both encodings
 bool gemv1_takes(const GemvP& p);                   // does one row's op run on gemv1.hip
 void launch_gemv1(const GemvP& p, hipStream_t s);   // one row, both encodings

@@ -356,6 +356,20 @@ def test_gemvM_long_split_in_k_slices(dev, M, N, K, pro, epi):
     assert np.array_equal(a[1].view(np.uint32), b[1].view(np.uint32))
 
 
+# gemvm_takes, on both sides of its lines: few rows with short splits of many blocks, and long splits
+@pytest.mark.parametrize("M,N,K,pro,epi,kPer", [
+    (2, 64, 64, "raw", "store", 0), (2, 64, 96, "raw", "store", 0), (2, 8192, 640, "rms", "store", 0),
+    (2, 8192, 672, "rms", "store", 0), (2, 4096, 320, "raw", "geglu", 0), (3, 8192, 256, "raw", "softcap", 0),
+    (3, 8192, 288, "raw", "store", 0), (3, 4160, 640, "rms", "geglu", 0), (4, 64, 8192, "raw", "store", 256),
+    (5, 64, 7936, "raw", "store", 256), (2, 4096, 4160, "raw", "store", 0), (2, 4160, 4128, "raw", "store", 0),
+    (3, 2112, 4128, "rms", "store", 0), (2, 8256, 2080, "rms", "geglu", 0), (3, 256, 2560, "rms", "softcap", 0),
+    (2, 4160, 2080, "rms", "softcap", 0),
+])
+def test_gemvM_few_rows_routes(dev, M, N, K, pro, epi, kPer):
+    Case(M, N, K, pro, epi, kPer=kPer, seed=20 + M, w_off=4, rowB=3, ldx=K + 5, ldm=N + 7, gemvM=True).check(
+        f"gemvM M={M} {N}x{K} {pro} {epi} kPer {kPer}")
+
+
 def one_row(N, K, pro, epi, kPer):
     Case(1, N, K, pro, epi, kPer=kPer, seed=70, w_off=4, rowB=3 if pro in ("raw", "rms") else 0, ldx=K + 5).check(
         f"gemv {N}x{K} {pro} {epi}")
