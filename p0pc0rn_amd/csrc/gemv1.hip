@@ -112,13 +112,16 @@ __global__ __launch_bounds__(kGmThreads) void gemv1_kernel(GmP p) {
 
   // ---- x' and its group sums
   float v[4] = {__uint_as_float(xv.x), __uint_as_float(xv.y), __uint_as_float(xv.z), __uint_as_float(xv.w)};
-  if (!plain)   // sum, pleg: the other partials, in order (engine/llm/lops.js:50-57)
-    for (int j = 1; j < p.nsrc; ++j) {
-      const u32x4 t = *P0_GLOBAL(const u32x4, p.X + j * p.ldp + kx);
-      v[0] += __uint_as_float(t.x);
-      v[1] += __uint_as_float(t.y);
-      v[2] += __uint_as_float(t.z);
-      v[3] += __uint_as_float(t.w);
+  if (!plain)   // sum, pleg: the other partials, in order (engine/llm/lops.js:50-57), four in flight; past the last: not added
+    for (int j = 1; j < p.nsrc; j += 4) {
+      u32x4 t[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) t[u] = *P0_GLOBAL(const u32x4, p.X + min(j + u, p.nsrc - 1) * p.ldp + kx);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (j + u < p.nsrc)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] += __uint_as_float(t[u][e]);
     }
   const float n[4] = {__uint_as_float(nv.x), __uint_as_float(nv.y), __uint_as_float(nv.z), __uint_as_float(nv.w)};
   float gs = 0.0f;
@@ -208,21 +211,34 @@ static void launch_enc(const GemvP& p, hipStream_t s) {
 
 // Splits of at most 2048 k (a wave's records of more do not fit its registers). A q4 op of more than 1024 tiles streams
 // from HBM on gemv.hip's kernel: 262144 x 2048 61.2 us there and 61.5 here, with a softcap 66.4 and 70.8; at 65536 rows
-// 20.8 and 18.9, 21.8 and 20.3
+// 20.3 and 17.8, 21.7 and 19.9
 //
 // A short split leaves most of a workgroup's 8 waves without records (a wave takes 128 k of a q4 row at a time, 64 of a
 // q8 row), which a call of several items per workgroup, or of a softcap's 4 blocks per item, pays for item by item: such
-// calls stay on gemv.hip's and gemv_q8.hip's kernels. Per recorded launch, us here / there: q4 geglu 16384 x 320 7.8 / 5.2,
-// x 960 9.5 / 8.4, x 1280 10.0 / 10.2, 4096 x 320 (512 blocks) 4.1 / 4.9; q4 store 16384 x 640 5.2 / 5.1, x 960 5.6 / 6.1,
-// 8192 x 320 4.0 / 4.6; q4 softcap 16384 x 640 6.1 / 5.8, x 960 6.7 / 6.8, 1024 x 320 5.4 / 5.0, x 960 5.5 / 6.2;
-// q8 geglu 16384 x 1024 11.3 / 11.0, 4096 x 320 4.8 / 6.3; q8 store 16384 x 320 6.0 / 5.3, x 640 6.6 / 7.3; q8 softcap
-// 4096 x 320 7.3 / 5.8, 16384 x 1024 8.9 / 8.7.
+// calls stay on gemv.hip's and gemv_q8.hip's kernels, from more k the more blocks there are. Per recorded launch, us here /
+// there: q4 store 8192 x 320 (512 blocks) 4.0 / 4.6, 16384 x 640 (1024) 5.2 / 5.1, x 960 5.6 / 6.1, 2560 x 10240 in 10 splits
+// (1600) 7.9 / 7.5, 8192 x 8192 in 8 (4096) 14.4 / 12.7, 65536 x 1024 14.3 / 12.1, x 1280 14.8 / 14.9; q4 geglu 4096 x 320
+// (512) 4.1 / 4.9, 16384 x 960 (2048) 9.5 / 8.4, x 1280 9.6 / 9.9, 32768 x 1280 (4096) 16.5 / 14.3, x 2048 20.5 / 18.6; q4
+// softcap 1024 x 320 5.4 / 5.0, 4096 x 704 (256) 5.2 / 5.5, 16384 x 704 (1024) 6.0 / 5.7, x 1024 6.3 / 6.4, 32768 x 704 8.5 /
+// 7.4, 65536 x 1024 (4096) 15.0 / 13.5, x 1280 16.1 / 16.3; q8 store 64 x 32768 in 128 splits (512) 4.7 / 4.0, 16384 x 320
+// 6.0 / 5.3, x 704 6.1 / 6.5, 32768 x 704 (2048) 10.3 / 8.1, x 1024 11.0 / 12.7; q8 geglu 4096 x 320 4.8 / 6.3, 16384 x 1024
+// 11.3 / 11.0; q8 softcap 4096 x 320 7.3 / 5.8, 16384 x 1024 8.9 / 8.7, 1024 x 2048 (64) 7.0 / 6.7, 4096 x 2048 7.2 / 8.2.
 bool gemv1_takes(const GemvP& p) {
   const bool q8 = p.enc == P0_ENC_Q8G64S_T64, geglu = p.epi == P0_EPI_GEGLU;
   if (p.kPer > kGmPass || (!q8 && p.NT > 1024)) return false;
-  if (p.epi == P0_EPI_SOFTCAP) return p.kPer > (q8 ? 1024 : 640);
   const int64_t blocks = (int64_t)(p.N / 16) * (geglu ? 2 : 1) * p.nsplit;
-  return blocks <= 512 || p.kPer >= (geglu ? (q8 ? 1088 : 1280) : (q8 ? 640 : 960));
+  if (p.epi == P0_EPI_SOFTCAP)
+    return q8 ? p.kPer > 1024 && blocks > 64 : p.kPer > (blocks <= 512 ? 640 : blocks <= 2048 ? 960 : 1152);
+  if (q8) {
+    // four groups are one each for gemv_q8.hip's four waves, which read partials and ev as they need them: 64 x 64 3.4 / 3.2,
+    // pleg 2048 x 256 over one partial 3.8 / 3.7, 64 x 256 over 4 4.0 / 3.8
+    if (p.kPer <= (p.pro == P0_PRO_SUM || p.pro == P0_PRO_PLEG ? 256 : 64)) return false;
+    if (blocks <= 512) return blocks <= 256 || p.kPer > 256;
+    return p.kPer >= (geglu ? 1088 : blocks <= 1024 ? 640 : 1024);
+  }
+  if (blocks <= 512) return true;
+  if (geglu) return blocks <= 2048 && p.kPer >= 1280;
+  return p.kPer >= (blocks <= 1024 ? 960 : 1152);
 }
 
 void launch_gemv1(const GemvP& p, hipStream_t s) {

@@ -400,9 +400,18 @@ def test_gemv_one_row_shapes(dev, N, K, pro, epi, kPer):
     (8192, 64, "rms", "store", 0), (8256, 928, "raw", "store", 0), (16448, 960, "rms", "store", 0),
     (4096, 64, "raw", "geglu", 0), (4160, 1248, "rms", "geglu", 0), (8256, 1280, "pleg", "geglu", 0),
     (64, 640, "rms", "softcap", 0), (8256, 672, "raw", "softcap", 0), (4160, 1888, "sum", "store", 960),
+    (8192, 672, "raw", "softcap", 0), (8256, 992, "rms", "softcap", 0), (32832, 1152, "raw", "softcap", 0),
+    (16448, 1152, "rms", "store", 0), (16448, 1120, "raw", "store", 0), (16448, 1280, "raw", "geglu", 0),
 ])
 def test_gemv_one_row_short_splits(dev, N, K, pro, epi, kPer):
     one_row(N, K, pro, epi, kPer)
+
+
+@pytest.mark.parametrize("pro", ["sum", "pleg"])
+@pytest.mark.parametrize("nsrc", [1, 2, 4, 5, 8, 9])
+def test_gemv_one_row_partials_in_fours(dev, pro, nsrc):
+    """the partials of a sum or pleg prologue are loaded four at a time behind the first: counts around multiples of four"""
+    Case(1, 128, 320, pro, "store", seed=70 + nsrc, ldx=325, nsrc=nsrc).check(f"gemv {pro} of {nsrc} partials")
 
 
 @pytest.mark.parametrize("scale", [1e-30, 1e-3, 1e4, 1e30])

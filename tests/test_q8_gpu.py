@@ -92,7 +92,12 @@ def test_q8_k_slices_across_workgroups(dev, slices, pro, epi, K, kPer):
     (4160, 1024, "rms", "geglu", 0),
     (8256, 1088, "rms", "geglu", 0),
     (8256, 576, "raw", "store", 0),
-    (16448, 640, "raw", "store", 0),
+    (16384, 640, "raw", "store", 0),
+    (16448, 960, "raw", "store", 0),
+    (16448, 1024, "rms", "store", 0),
+    (8192, 256, "raw", "store", 0),
+    (8192, 320, "rms", "store", 0),
+    (1024, 1088, "raw", "softcap", 0),
 ])
 def test_q8_one_row_shapes(dev, N, K, pro, epi, kPer):
     """gemv1.hip's q8 form where its pieces end, and the splits past its rule; the bar of the file's gemvM test"""
