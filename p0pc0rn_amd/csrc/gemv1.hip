@@ -15,7 +15,8 @@
 // 2048 x 2048 5.8 -> 3.2, 2048 x 8192 in 4 splits 7.0 -> 4.9, 256 x 2048 5.2 -> 2.8, 65536 x 2048 20.8 -> 18.9; q8 5120 x
 // 1536 6.9 -> 5.0, 1536 x 6144 in 3 splits 7.6 -> 5.4, geglu 6144 x 1536 9.1 -> 7.1 and 12288 x 1536 11.4 -> 10.3, 65536 x
 // 1536 30.3 -> 23.8. Relative L2 against float64: q4 1.9e-7 - 2.7e-7 (1.9e-7 - 2.8e-7 before), q8 2.0e-7 (3.8e-7).
-// Tried: items of 4 blocks (q8 geglu 12288 12.5 us: 192 workgroups of 2 items), 2 workgroups per CU (65536 x 2048 18.6,
+// Tried: the partials of a sum or pleg four at a time (q4 over 16 4.3 -> 3.9 us, but every q8 call 0.2 us slower), items of
+// 4 blocks (q8 geglu 12288 12.5 us: 192 workgroups of 2 items), 2 workgroups per CU (65536 x 2048 18.6,
 // but q8 geglu 6144 8.9), the next item's records loaded block by block as registers come free (262144 x 2048 76 us).
 #include "gemvm.hpp"
 
@@ -112,16 +113,13 @@ __global__ __launch_bounds__(kGmThreads) void gemv1_kernel(GmP p) {
 
   // ---- x' and its group sums
   float v[4] = {__uint_as_float(xv.x), __uint_as_float(xv.y), __uint_as_float(xv.z), __uint_as_float(xv.w)};
-  if (!plain)   // sum, pleg: the other partials, in order (engine/llm/lops.js:50-57), four in flight; past the last: not added
-    for (int j = 1; j < p.nsrc; j += 4) {
-      u32x4 t[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) t[u] = *P0_GLOBAL(const u32x4, p.X + min(j + u, p.nsrc - 1) * p.ldp + kx);
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (j + u < p.nsrc)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] += __uint_as_float(t[u][e]);
+  if (!plain)   // sum, pleg: the other partials, in order (engine/llm/lops.js:50-57)
+    for (int j = 1; j < p.nsrc; ++j) {
+      const u32x4 t = *P0_GLOBAL(const u32x4, p.X + j * p.ldp + kx);
+      v[0] += __uint_as_float(t.x);
+      v[1] += __uint_as_float(t.y);
+      v[2] += __uint_as_float(t.z);
+      v[3] += __uint_as_float(t.w);
     }
   const float n[4] = {__uint_as_float(nv.x), __uint_as_float(nv.y), __uint_as_float(nv.z), __uint_as_float(nv.w)};
   float gs = 0.0f;
@@ -230,9 +228,9 @@ bool gemv1_takes(const GemvP& p) {
   if (p.epi == P0_EPI_SOFTCAP)
     return q8 ? p.kPer > 1024 && blocks > 64 : p.kPer > (blocks <= 512 ? 640 : blocks <= 2048 ? 960 : 1152);
   if (q8) {
-    // four groups are one each for gemv_q8.hip's four waves, which read partials and ev as they need them: 64 x 64 3.4 / 3.2,
-    // pleg 2048 x 256 over one partial 3.8 / 3.7, 64 x 256 over 4 4.0 / 3.8
-    if (p.kPer <= (p.pro == P0_PRO_SUM || p.pro == P0_PRO_PLEG ? 256 : 64)) return false;
+    // four groups are one each for gemv_q8.hip's four waves, which read the partials as they need them: pleg 64 x 256 over
+    // one partial 3.4 / 3.5, over 4 3.9 / 3.7, over 16 5.1 / 4.7
+    if (p.kPer <= 256 && p.nsrc > 1 && (p.pro == P0_PRO_SUM || p.pro == P0_PRO_PLEG)) return false;
     if (blocks <= 512) return blocks <= 256 || p.kPer > 256;
     return p.kPer >= (geglu ? 1088 : blocks <= 1024 ? 640 : 1024);
   }
