@@ -49,6 +49,7 @@ Ctx& ctx();
 int ensure_xstage(size_t bytes, const char* op);   // P0_OK, or an error (no room while the stream is being captured)
 // per-file set-up at p0_open (kernel attributes; the no-allocation GEMM's scratch address)
 int gemm_init();
+int misc_init();
 
 // Thread-local message of the last failure (p0_last_error).
 void set_error(const char* fmt, ...) __attribute__((format(printf, 1, 2)));

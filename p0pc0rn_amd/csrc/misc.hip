@@ -3,11 +3,12 @@
 // writes. rowstats and normadd sum in the reference's order (256 partials, partial t over elements t, t + 256, ... in
 // turn, then a halving tree), so the fp32 sums equal the reference's, bit for bit.
 //
-// One wave owns a row: lane l holds the partials 4 l .. 4 l + 3, so 256 consecutive elements are one 16-byte load per
-// lane, and the whole tree is lane moves within the wave (no LDS, no barrier). Bound: at a decode step's one row, the
-// memory round trips (launch, loads, stores); at thousands of rows, HBM bandwidth. A workgroup of 256 threads per row
-// with one 4-byte load in flight per thread and nine barriers a tree took, per launch, 11.5 us for a normadd of 2048
-// values over 1 or 4 partials and 24.7 us for the statistics of 4608 x 3072 values; this takes 4.1 and 11.7 (4.9 TB/s).
+// Rows of 16-byte aligned values: one wave owns a row, lane l holds the partials 4 l .. 4 l + 3, so 256 consecutive elements
+// are one 16-byte load per lane, and the whole tree is lane moves within the wave (no LDS, no barrier). Bound: at a decode
+// step's one row, the memory round trips (launch, loads, stores); at thousands of rows, HBM bandwidth. A workgroup of 256
+// threads per row with one 4-byte load in flight per thread and nine barriers a tree took, per recorded launch, 24.7 us for
+// the statistics of 4608 x 3072 values; this takes 11.7 (4.9 TB/s). Rows that are not aligned, and normadds of lengths that
+// suit no form of the wave's, are still a workgroup's.
 #include "common.hpp"
 
 // no FMA contraction: every a + b * c rounds the product and the sum separately, as the CPU restatement does, so the
@@ -41,6 +42,22 @@ __device__ __forceinline__ float tree256(const float (&part)[4]) {
     v[c] = t + dpp_move<0x121>(t);
   }
   return (v[0] + v[2]) + (v[1] + v[3]);
+}
+
+// the same tree over 256 threads' partials through LDS
+constexpr int kRowThreads = 256;
+__device__ __forceinline__ float tree256_lds(float v, float* red) {
+  const int t = threadIdx.x;
+  red[t] = v;
+  __syncthreads();
+#pragma unroll
+  for (int s = 128; s > 0; s >>= 1) {
+    if (t < s) red[t] = red[t] + red[t + s];
+    __syncthreads();
+  }
+  const float r = red[0];
+  __syncthreads();
+  return r;
 }
 
 __device__ __forceinline__ float rsqrt_exact(float v) { return 1.0f / __builtin_sqrtf(v); }
@@ -120,10 +137,10 @@ __global__ __launch_bounds__(256) void rowstats_kernel(const float* __restrict__
   }
 }
 
-// engine/llm/lops.js:153-170. ONCE: the row's partials (four at a time), its residual and the norm weights are all in
-// flight together before the first sum; longer rows add the partials again in the second pass (the same order, the
-// same bits).
-template <bool VEC, int NB, bool ONCE>
+// engine/llm/lops.js:153-170, 16-byte aligned rows, a wave a row. ONCE: the row's partials (four at a time), its residual and
+// the norm weights are all in flight together before the first sum; longer rows add the partials again in the second
+// pass (the same order, the same bits).
+template <int NB, bool ONCE>
 __global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T, int64_t nsrc, int64_t ldp,
                                                      const float* __restrict__ W, int64_t woff, float* X,
                                                      float* __restrict__ ST, int64_t stoff, int64_t D, float eps,
@@ -151,14 +168,14 @@ __global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int k = 0; k < NB; ++k) v[u][k] = load4<VEC>(T + (j + u) * ldp + xb + b, k * kChunk + 4 * lane, n);
+        for (int k = 0; k < NB; ++k) v[u][k] = load4<true>(T + (j + u) * ldp + xb + b, k * kChunk + 4 * lane, n);
 #pragma unroll
       for (int u = 0; u < 4; ++u) add(v[u]);
     }
     for (; j < nsrc; ++j) {
       float4 v[NB];
 #pragma unroll
-      for (int k = 0; k < NB; ++k) v[k] = load4<VEC>(T + j * ldp + xb + b, k * kChunk + 4 * lane, n);
+      for (int k = 0; k < NB; ++k) v[k] = load4<true>(T + j * ldp + xb + b, k * kChunk + 4 * lane, n);
       add(v);
     }
   };
@@ -168,8 +185,8 @@ __global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T
     for (int k = 0; k < NB; ++k) {
       xv[k] = wv[k] = float4{0.0f, 0.0f, 0.0f, 0.0f};
       if (mode == 0) {
-        xv[k] = load4<VEC>(X + xb + b, k * kChunk + 4 * lane, n);
-        wv[k] = load4<VEC>(W + woff + b, k * kChunk + 4 * lane, n);
+        xv[k] = load4<true>(X + xb + b, k * kChunk + 4 * lane, n);
+        wv[k] = load4<true>(W + woff + b, k * kChunk + 4 * lane, n);
       }
     }
   };
@@ -200,15 +217,9 @@ __global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         y[c] = mode == 0 ? (at(xv[k], c) + at(t[k], c) * rs * at(wv[k], c)) * scale : at(t[k], c);
-        s2[c] = i + (VEC ? 0 : c) < n ? s2[c] + y[c] * y[c] : s2[c];
+        s2[c] = i < n ? s2[c] + y[c] * y[c] : s2[c];
       }
-      if (VEC) {
-        if (i < n) *(float4*)(X + xb + b + i) = float4{y[0], y[1], y[2], y[3]};
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (i + c < n) X[xb + b + i + c] = y[c];
-      }
+      if (i < n) *(float4*)(X + xb + b + i) = float4{y[0], y[1], y[2], y[3]};
     }
   };
   if (ONCE) {
@@ -222,6 +233,35 @@ __global__ __launch_bounds__(64) void normadd_kernel(const float* __restrict__ T
   }
   const float r2 = tree256(s2);
   if (lane == 0) ST[stoff + m] = rsqrt_exact(r2 / (float)D + eps);
+}
+
+// The same for any row: 256 threads, one element each at a time, the row's sums in LDS between the passes (D floats).
+__global__ __launch_bounds__(kRowThreads) void normadd_any_kernel(const float* __restrict__ T, int64_t nsrc, int64_t ldp,
+                                                                  const float* __restrict__ W, int64_t woff, float* X,
+                                                                  float* __restrict__ ST, int64_t stoff, int64_t D, float eps,
+                                                                  float scale, int mode) {
+  __shared__ float red[kRowThreads];
+  extern __shared__ float tv[];
+  const int t = threadIdx.x;
+  const int64_t m = blockIdx.x, xb = m * D;
+  float s = 0.0f;
+  for (int64_t i = t; i < D; i += kRowThreads) {
+    float v = 0.0f;
+    for (int64_t j = 0; j < nsrc; ++j) v = v + T[j * ldp + xb + i];
+    tv[i] = v;
+    s = s + v * v;
+  }
+  const float rs = rsqrt_exact(tree256_lds(s, red) / (float)D + eps);
+  float s2 = 0.0f;
+  for (int64_t i = t; i < D; i += kRowThreads) {
+    float x = X[xb + i];
+    if (mode == 0) x = (x + tv[i] * rs * W[woff + i]) * scale;
+    else x = tv[i];
+    X[xb + i] = x;
+    s2 = s2 + x * x;
+  }
+  const float r2 = tree256_lds(s2, red);
+  if (t == 0) ST[stoff + m] = rsqrt_exact(r2 / (float)D + eps);
 }
 
 // The same for rows of at most 2048 values, 16-byte aligned, and few of them (a decode step's, a verify pass's): a wave per
@@ -331,6 +371,13 @@ __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const float* __rest
   }
 }
 
+// normadd's LDS allowance (one row of up to 150 KB), set once at p0_open
+int misc_init() {
+  P0_HIP(hipFuncSetAttribute((const void*)normadd_any_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024),
+         "p0_open: normadd");
+  return P0_OK;
+}
+
 static bool vec_ok(const float* p, int64_t a, int64_t b) { return (((uintptr_t)p | (uintptr_t)(a * 4) | (uintptr_t)(b * 4)) & 15) == 0; }
 
 }  // namespace p0
@@ -373,7 +420,9 @@ extern "C" int p0_normadd(const p0_normadd_args_t* a) {
   if (D <= 0 || M < 0) { set_error("normadd: D %lld, M %lld", (long long)D, (long long)M); return P0_EINVAL; }
   if (a->mode != 0 && a->mode != 1) { set_error("normadd: mode %d", (int)a->mode); return P0_EINVAL; }
   if (!a->t || !a->x || !a->st || (a->mode == 0 && !a->w)) { set_error("normadd: missing t, w, x or st buffer"); return P0_EINVAL; }
-  if (D * (int64_t)sizeof(float) > 150 * 1024) { set_error("normadd: D %lld exceeds this build's row buffer", (long long)D); return P0_EINVAL; }
+  if (D * (int64_t)sizeof(float) > 150 * 1024) {   // normadd_any_kernel's row in LDS
+    set_error("normadd: D %lld exceeds this build's row buffer", (long long)D); return P0_EINVAL;
+  }
   if (int r = require_open("normadd")) return r;
   const int64_t nsrc = a->t_n ? a->t_n : 1, ldp = a->t_ld ? a->t_ld : D * M;
   const float eps = a->eps != 0.0f ? a->eps : 1e-6f;
@@ -386,9 +435,18 @@ extern "C" int p0_normadd(const p0_normadd_args_t* a) {
     P0_LAUNCHED("normadd");
     return P0_OK;
   }
-  auto k = !vec ? normadd_kernel<false, 4, false> : D <= 8 * kChunk ? normadd_kernel<true, 8, true> : normadd_kernel<true, 8, false>;
-  hipLaunchKernelGGL(k, dim3((unsigned)M), dim3(64), 0, ctx().cur, a->t, nsrc, ldp, a->w,
-                     a->w_off, a->x, a->st, a->st_off, D, eps, a->scale, (int)a->mode);
+  // a wave a row where it holds the row and there is enough of it (us, a wave / a workgroup a row: 4608 rows of 512 over one
+  // partial 10.1 / 9.8, of 768 10.6 / 12.8, 512 rows of 256 4.5 / 4.1), or in batches of 2048 from 3072 on (one row of 2304
+  // 6.6 / 5.8, of 4096 6.8 / 7.9; 4608 rows of 2304 36.0 / 28.7, of 4096 40 / 45); rows that are not 16-byte aligned take a
+  // workgroup each (one row of 2048 7.0 / 5.4, 4608 rows 46 / 27)
+  if (vec && (D >= 3072 || (D >= 768 && D <= 8 * kChunk))) {
+    auto k = D <= 8 * kChunk ? normadd_kernel<8, true> : normadd_kernel<8, false>;
+    hipLaunchKernelGGL(k, dim3((unsigned)M), dim3(64), 0, ctx().cur, a->t, nsrc, ldp, a->w, a->w_off, a->x, a->st, a->st_off, D,
+                       eps, a->scale, (int)a->mode);
+  } else {
+    hipLaunchKernelGGL(normadd_any_kernel, dim3((unsigned)M), dim3(kRowThreads), (size_t)D * sizeof(float), ctx().cur, a->t,
+                       nsrc, ldp, a->w, a->w_off, a->x, a->st, a->st_off, D, eps, a->scale, (int)a->mode);
+  }
   P0_LAUNCHED("normadd");
   return P0_OK;
 }

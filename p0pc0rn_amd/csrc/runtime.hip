@@ -136,6 +136,7 @@ int p0_open(int device) {
   P0_HIP(hipMemset(c.counters, 0, kAllCounters * sizeof(unsigned)), "p0_open: workspace");
   P0_HIP(hipDeviceSynchronize(), "p0_open");
   if (int r = gemm_init()) return r;
+  if (int r = misc_init()) return r;
   c.part_floats = kPartBytes / sizeof(float);
   c.n_counters = kCounters;
   c.gemm_counters = c.counters + kCounters;

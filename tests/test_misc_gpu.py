@@ -130,3 +130,31 @@ def test_normadd_aligned_rows_bit_exact(dev, D, M, nsrc, mode):
     assert np.array_equal(gs, sw.view(np.uint32))
     for b in (tb, wb, xb, sb):
         b.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("D,M,nsrc,ldp_pad,w_off,shift", [
+    (1, 3, 1, 1, 0, 0), (3, 2, 4, 5, 1, 1), (255, 300, 2, 1, 1, 0), (1027, 2, 3, 7, 0, 1), (2050, 1, 5, 0, 1, 0),
+    (2048, 5, 4, 0, 0, 1), (2048, 2, 1, 0, 1, 0), (8193, 1, 2, 3, 3, 1), (38400, 1, 1, 1, 0, 0),
+    (764, 257, 1, 0, 0, 0), (768, 257, 3, 0, 0, 0), (2048, 257, 2, 0, 0, 0), (3068, 2, 1, 0, 0, 0), (3072, 2, 5, 0, 0, 0),
+])
+def test_normadd_any_rows_bit_exact(dev, D, M, nsrc, ldp_pad, w_off, shift, mode):
+    """rows, strides and buffers at any alignment, and both sides of the sizes where aligned rows take a wave or a workgroup
+    each; nothing past x written"""
+    ldp = M * D + ldp_pad
+    t = O.randn(nsrc * ldp + 1, D + nsrc, 0.3).astype(np.float32)
+    w = (0.5 + O.rng_uniform(D, D + w_off)).astype(np.float32)
+    x0 = O.randn(M * D, D + 1).astype(np.float32)
+    xw, sw = x0.copy(), np.full(M, np.nan, np.float32)
+    kw = dict(t_n=nsrc, t_ld=ldp, w_off=w_off, D=D, M=M, eps=1e-6, scale=0.9, mode=mode)
+    O.normadd(capi.normadd_args(t=t.ctypes.data, w=w.ctypes.data, x=xw.ctypes.data, st=sw.ctypes.data, **kw))
+    tb, wb, xb = capi.to_device(t), capi.to_device(w), capi.Buffer(x0.nbytes + 32).fill_u32(NAN)
+    xb.upload(x0, 4 * shift)
+    sb = capi.Buffer(sw.nbytes).fill_u32(NAN)
+    capi.normadd(capi.normadd_args(t=tb, w=wb, x=xb.ptr + 4 * shift, st=sb, **kw))
+    gx, gs = xb.read(np.float32).view(np.uint32), sb.read(np.float32, M).view(np.uint32)
+    assert np.array_equal(gx[shift:M * D + shift], xw.view(np.uint32))
+    assert (gx[:shift] == NAN).all() and (gx[M * D + shift:M * D + 8] == NAN).all()
+    assert np.array_equal(gs, sw.view(np.uint32))
+    for b in (tb, wb, xb, sb):
+        b.free()
