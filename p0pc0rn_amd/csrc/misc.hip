@@ -137,6 +137,33 @@ __global__ __launch_bounds__(256) void rowstats_kernel(const float* __restrict__
   }
 }
 
+// The same for any row, 256 threads a row, one element each at a time.
+__global__ __launch_bounds__(kRowThreads) void rowstats_any_kernel(const float* __restrict__ x, int64_t ld, int64_t c0,
+                                                                   int64_t rows, int64_t cols, int mode, float eps,
+                                                                   float* __restrict__ st, int64_t st_off) {
+  __shared__ float red[kRowThreads];
+  const int t = threadIdx.x;
+  for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    const float* xr = x + row * ld + c0;
+    float mean = 0.0f;
+    if (mode == 0) {
+      float s = 0.0f;
+      for (int64_t i = t; i < cols; i += kRowThreads) s = s + xr[i];
+      mean = tree256_lds(s, red) / (float)cols;
+    }
+    float q = 0.0f;
+    for (int64_t i = t; i < cols; i += kRowThreads) {
+      const float d = xr[i] - mean;
+      q = q + d * d;
+    }
+    const float var = tree256_lds(q, red) / (float)cols;
+    if (t == 0) {
+      st[(st_off + row) * 2] = mean;
+      st[(st_off + row) * 2 + 1] = rsqrt_exact(var + eps);
+    }
+  }
+}
+
 // engine/llm/lops.js:153-170, 16-byte aligned rows, a wave a row. ONCE: the row's partials (four at a time), its residual and
 // the norm weights are all in flight together before the first sum; longer rows add the partials again in the second
 // pass (the same order, the same bits).
@@ -404,6 +431,16 @@ extern "C" int p0_rowstats(const p0_rowstats_args_t* a) {
   const int64_t blocks = (a->rows + wpb - 1) / wpb;
   const unsigned grid = (unsigned)(blocks < 65536 * 4 ? blocks : 65536 * 4);
   const bool vec = vec_ok(x, ld, a->x_c0) && a->cols % 4 == 0;
+  // rows that are not 16-byte aligned are four 4-byte loads a lane and 256 values: a workgroup a row wins from 4096 columns,
+  // or 512 once the rows fill the chip (mean and variance, us, a wave / a workgroup a row: one row of 3071 4.9 / 5.0, of 4099
+  // 6.7 / 5.7; 1024 rows of 511 3.8 / 4.2, of 2047 6.5 / 5.4; 4608 rows of 2047 20.9 / 16.9)
+  if (!vec && a->cols > (a->rows <= 256 ? 4096 : 512)) {
+    const unsigned g = (unsigned)(a->rows < 65536 * 4 ? a->rows : 65536 * 4);
+    hipLaunchKernelGGL(rowstats_any_kernel, dim3(g), dim3(kRowThreads), 0, ctx().cur, x, ld, a->x_c0, a->rows, a->cols,
+                       (int)a->mode, a->eps, a->st, a->st_off);
+    P0_LAUNCHED("rowstats");
+    return P0_OK;
+  }
   auto k = !vec                       ? rowstats_kernel<false, 4, false>
            : a->cols <= 8 * kChunk    ? rowstats_kernel<true, 8, true>
            : a->cols <= 16 * kChunk   ? rowstats_kernel<true, 16, true>

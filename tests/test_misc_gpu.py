@@ -158,3 +158,10 @@ def test_normadd_any_rows_bit_exact(dev, D, M, nsrc, ldp_pad, w_off, shift, mode
     assert np.array_equal(gs, sw.view(np.uint32))
     for b in (tb, wb, xb, sb):
         b.free()
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("rows,cols", [(1, 4095), (2, 4097), (256, 4096), (257, 511), (257, 513), (1030, 515)])
+def test_rowstats_unaligned_rows_bit_exact(dev, rows, cols, mode):
+    """rows that are not 16-byte aligned, on both sides of the sizes where a row takes a wave or a workgroup"""
+    test_rowstats_bit_exact(dev, rows, cols, mode)
