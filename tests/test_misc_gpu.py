@@ -91,6 +91,12 @@ def test_argmax_of_a_softcap_gemv(dev):
         b.free()
 
 
+@pytest.mark.parametrize("n,M", [(1024, 1), (1025, 1), (1025, 171), (1026, 171), (1023, 700), (255, 1030), (9000, 2)])
+def test_argmax_exact_wave_counts(dev, n, M):
+    """both workgroup sizes: on both sides of 1024 pairs and of 6 pairs per row"""
+    test_argmax_exact(dev, n, M)
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 @pytest.mark.parametrize("rows,cols", [(1, 4), (5, 252), (1027, 256), (3, 2048), (2, 2052), (5, 4096), (2, 4100), (1, 9000)])
 def test_rowstats_aligned_rows_bit_exact(dev, rows, cols, mode):
