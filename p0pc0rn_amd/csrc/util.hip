@@ -7,8 +7,8 @@ typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
 
 // A workgroup takes one 64-row tile x 8 groups: its 8 records (10 KB) go through LDS as they lie in memory, so that the
 // reads are whole records and each row's 256 values leave as 512 (1024) consecutive bytes. Bound: HBM, 0.625 B read and
-// 2 or 4 B written per weight. 9216 x 3072 to fp16: 12.2 us (6.1 TB/s); a thread per (row, code word) with 2-byte stores
-// and a 64-bit division per word took 40.5.
+// 2 or 4 B written per weight. 9216 x 3072 to fp16: 12.2 us again and again over the same 74 MB, which then stay in the
+// last-level cache (40.5 with the kernel below), 26 over a weight and an output not touched before (54).
 // fl32(q * s + m) as engine/kcheck.js:32 / engine/core/store.js:291 compute it (q * s is exact in f32, so the fused and
 // unfused forms round the same), and fl16 of that as the GEMM tile (engine/ops/gemm.js:147-148).
 constexpr int kDqGroups = 8, kDqRec = 324;   // words per record in LDS: 320, + 4 so that records start on other banks
@@ -70,6 +70,27 @@ __global__ __launch_bounds__(256) void q4_dequant_kernel(const uint8_t* __restri
   }
 }
 
+// The same for small weights: a thread per (row, code word), the 8 weights k = 32 g + 8 w .. + 7 of row n.
+__global__ void q4_dequant_words_kernel(const uint8_t* __restrict__ w, int64_t wG, int64_t N, int64_t K,
+                                        float* __restrict__ o32, uint16_t* __restrict__ o16) {
+  const int64_t words = N * (K / 8);
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t n = i / (K / 8), kw = i - n * (K / 8), g = kw >> 2, wd = kw & 3;
+    const uint8_t* rec = w + ((n >> 6) * wG + g) * 1280;
+    const int r = (int)(n & 63);
+    const uint32_t q = *(const uint32_t*)(rec + r * 16 + wd * 4);
+    const h2_t sm = __builtin_bit_cast(h2_t, *(const uint32_t*)(rec + 1024 + r * 4));
+    const float s = (float)sm.x, m = (float)sm.y;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float v = (float)((q >> (4 * j)) & 15u) * s + m;
+      const int64_t o = n * K + kw * 8 + j;
+      if (o32) o32[o] = v;
+      if (o16) o16[o] = __builtin_bit_cast(uint16_t, (_Float16)v);
+    }
+  }
+}
+
 // The PCG RXS-M-XS hash (Jarzynski & Olano, JCGT 2020), as the reference's GPU filler (engine/tune/autotune.js:76).
 __device__ __forceinline__ uint32_t hash32(uint32_t x) {
   uint32_t v = x * 747796405u + 2891336453u;
@@ -124,6 +145,14 @@ extern "C" int p0_q4_dequant(const void* w, int64_t w_off, int64_t N, int64_t K,
   if (w_off % 4) { set_error("dequant: weight offset"); return P0_EINVAL; }
   if (!w || (!out32 && !out16)) { set_error("dequant: missing buffer"); return P0_EINVAL; }
   if (int r = require_open("dequant")) return r;
+  // small weights have too few tiles for the chip: to fp16 256 x 256 3.9 us in tiles, 2.9 a word a thread, 1024 x 1024 4.2 /
+  // 3.8, 1024 x 2048 4.5 / 5.3; to fp32 512 x 1024 4.3 / 3.8, 1024 x 1024 4.9 / 5.0
+  if (N * K <= (out32 ? 1 << 19 : 5 << 18)) {
+    hipLaunchKernelGGL(q4_dequant_words_kernel, dim3(grid_for(N * K / 8)), dim3(256), 0, ctx().cur, (const uint8_t*)w + w_off,
+                       K / 32, N, K, out32, out16);
+    P0_LAUNCHED("dequant");
+    return P0_OK;
+  }
   const int64_t items = N / 64 * ((K / 32 + kDqGroups - 1) / kDqGroups);
   const bool vec = (((uintptr_t)out32 | (uintptr_t)out16) & 15) == 0;
   auto k = vec ? q4_dequant_kernel<true> : q4_dequant_kernel<false>;

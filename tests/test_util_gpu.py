@@ -114,9 +114,10 @@ def test_probe_read_reads_the_whole_buffer(dev):
 
 
 @pytest.mark.parametrize("shift", [0, 1])
-@pytest.mark.parametrize("N,K", [(64, 32), (128, 256), (64, 288), (192, 1056)])
+@pytest.mark.parametrize("N,K", [(64, 32), (128, 256), (64, 288), (192, 1056), (512, 2592), (640, 2080)])
 def test_dequant_group_remainders_and_alignment(dev, N, K, shift):
-    """a last block of fewer than 8 groups, and outputs that are not 16-byte aligned; nothing past the outputs written"""
+    """a last block of fewer than 8 groups, and outputs that are not 16-byte aligned; nothing past the outputs written. Small
+    weights a code word a thread, the last two in tiles"""
     b, _ = O.pack_q4(O.randn(N * K, N + K, 0.05), N, K)
     wb = capi.to_device(b)
     o32, o16 = capi.Buffer(4 * N * K + 32).fill_u32(0x7FC00000), capi.Buffer(2 * N * K + 32).fill_u32(0x7FC07FC0)
@@ -128,4 +129,18 @@ def test_dequant_group_remainders_and_alignment(dev, N, K, shift):
     assert np.array_equal(g16[shift:n + shift], np.asarray(w16).ravel().view(np.uint16))
     assert (g32[n + shift:n + 4] == 0x7FC00000).all() and (g16[n + 2:n + 8] == (0x7FC0)).all()
     for x in (wb, o32, o16):
+        x.free()
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("N,K", [(512, 1024), (512, 1056), (640, 2048), (640, 2080)])
+def test_dequant_one_output_sizes(dev, N, K, f32):
+    """one output alone, on both sides of the sizes from which a weight is taken in tiles (2^19 values to fp32, 5 * 2^18 to
+    fp16)"""
+    b, _ = O.pack_q4(O.randn(N * K, N + K, 0.05), N, K)
+    wb, out = capi.to_device(b), capi.Buffer((4 if f32 else 2) * N * K)
+    capi.q4_dequant(wb, N, K, **{"out32" if f32 else "out16": out})
+    want = np.asarray(O.dequant_q4(b, N, K)[0 if f32 else 1]).ravel()
+    assert np.array_equal(out.read(np.uint32 if f32 else np.uint16), want.view(np.uint32 if f32 else np.uint16))
+    for x in (wb, out):
         x.free()
