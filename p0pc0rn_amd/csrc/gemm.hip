@@ -44,18 +44,19 @@ __device__ __forceinline__ int swz_key(int r) { return (r ^ ((r >> 3) & 3)) & 7;
 __device__ __forceinline__ int swz(int r, int c) { return r * 128 + ((c ^ swz_key(r)) << 4); }
 
 // ------------------------------------------------------------------------------------------------ X staging
-// Bound: HBM, one read of X and one write of X'. A wave owns a strip of 512 columns (8 per lane: a 16-byte store, one or
-// two 16-byte loads) and walks `rpw` rows down it, UR rows' loads in flight, so that the modulation vectors of an lnmod
-// are loaded once per strip and no index is divided. 4608 x 3072, lnmod: 59 -> 14.5 us, 5.9 TB/s (one chunk of 8 per thread with a
-// 64-bit division and 16 scalar modulation loads each, before).
-constexpr int kStripCols = 512;
+// Bound: HBM, one read of X and one write of X'. A wave owns a strip of 8 L columns (8 per lane: a 16-byte store, one or
+// two 16-byte loads; L = 1 << ls lanes a row, 64 unless that would leave more than an eighth of them past K) of 64 / L rows
+// side by side and walks `rpw` such steps down it, UR steps' loads in flight, so that the modulation vectors of an lnmod
+// are loaded once per strip and no index is divided. 4608 x 3072, lnmod: 59 -> 14.5 us, 5.9 TB/s (one chunk of 8 per thread
+// with a 64-bit division and 16 scalar modulation loads each, before). With 64 lanes a row always, the calls of 65536 rows
+// of 32 columns took 24.4 us (the whole GEMM, bf16; 20.0 before) and of 544 57.9 (50.2).
 template <int MODE, int UR>
-__global__ __launch_bounds__(256) void x_stage_kernel(XStageP p, int rpw, int strips) {
-  const int lane = threadIdx.x & 63, rblk = blockIdx.x / strips;
-  const int k = (blockIdx.x - rblk * strips) * kStripCols + lane * 8;
-  if (k >= p.K) return;
-  const int64_t first = ((int64_t)rblk * 4 + (threadIdx.x >> 6)) * rpw;
-  const int r0 = (int)(first < p.M ? first : p.M), r1 = (int)(first + rpw < p.M ? first + rpw : p.M);
+__global__ __launch_bounds__(256) void x_stage_kernel(XStageP p, int rpw, int strips, int ls) {
+  const int lane = threadIdx.x & 63, rblk = blockIdx.x / strips, side = 64 >> ls;
+  const int k = (((blockIdx.x - rblk * strips) << ls) + (lane & ((1 << ls) - 1))) * 8;
+  const int64_t first = ((int64_t)rblk * 4 + (threadIdx.x >> 6)) * rpw * side + (lane >> ls);
+  if (k >= p.K || first >= p.M) return;
+  const int r0 = (int)first, r1 = (int)(first + (int64_t)rpw * side < p.M ? first + (int64_t)rpw * side : p.M);
   constexpr bool F32 = MODE == P0_XMODE_LNMOD || MODE == P0_XMODE_RMS;
   float sc[8], sh[8];   // lnmod: 1 + scale and shift; rms: the norm weights
   if (F32) {
@@ -69,13 +70,13 @@ __global__ __launch_bounds__(256) void x_stage_kernel(XStageP p, int rpw, int st
       }
     }
   }
-  for (int r = r0; r < r1; r += UR) {
+  for (int64_t r = r0; r < r1; r += UR * side) {
     u32x4n d[UR][F32 ? 2 : 1];
     float mean[UR], rstd[UR];
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
-      const int m = min(r + u, r1 - 1);
-      const int64_t idx = (int64_t)m * p.ldx + p.kx0 + k;
+      const int64_t m = r + u * side < r1 ? r + u * side : r;   // past the last: this step's first again (not stored)
+      const int64_t idx = m * p.ldx + p.kx0 + k;
       if (F32) {
         const float* src = (const float*)p.x + idx;
         mean[u] = p.st[(p.stOff + m) * 2];
@@ -102,7 +103,7 @@ __global__ __launch_bounds__(256) void x_stage_kernel(XStageP p, int rpw, int st
     }
 #pragma unroll
     for (int u = 0; u < UR; ++u) {
-      if (r + u >= r1) break;
+      if (r + u * side >= r1) break;
       float f[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
@@ -117,22 +118,25 @@ __global__ __launch_bounds__(256) void x_stage_kernel(XStageP p, int rpw, int st
       u32x4n o;
 #pragma unroll
       for (int i = 0; i < 4; ++i) o[i] = pack_h2(f[2 * i], f[2 * i + 1]);
-      *(u32x4n*)(p.out + (int64_t)(r + u) * p.K + k) = o;
+      *(u32x4n*)(p.out + (r + u * side) * p.K + k) = o;
     }
   }
 }
 
-// rows a wave walks: one while that gives the chip no more than 8 waves per SIMD (8192 in all), up to 8 beyond
+// steps a wave walks: one while that gives the chip no more than 8 waves per SIMD (8192 in all), up to 8 beyond
 static void launch_x_stage(const XStageP& q, hipStream_t s) {
-  const int strips = (q.K + kStripCols - 1) / kStripCols;
-  const int64_t waves = (int64_t)strips * q.M;
+  const int chunks = q.K / 8;   // a multiple of 4
+  int ls = 6;
+  while (((chunks + (1 << ls) - 1) >> ls << ls) - chunks > chunks / 8) --ls;   // 4 lanes always fit
+  const int strips = (chunks + (1 << ls) - 1) >> ls, side = 64 >> ls;
+  const int64_t steps = ((int64_t)q.M + side - 1) / side, waves = (int64_t)strips * steps;
   int rpw = waves <= 8192 ? 1 : waves <= 32768 ? 4 : 8;
   while (waves / rpw > (1 << 25)) rpw *= 2;   // a grid of at most 2^32 threads
-  const dim3 grid((unsigned)(((int64_t)q.M + 4 * rpw - 1) / (4 * rpw) * strips));
+  const dim3 grid((unsigned)((steps + 4 * rpw - 1) / (4 * rpw) * strips));
 #define P0_STAGE(MODE)                                                                          \
   if (q.xmode == MODE) {                                                                        \
     auto k = rpw == 1 ? x_stage_kernel<MODE, 1> : x_stage_kernel<MODE, 4>;                      \
-    hipLaunchKernelGGL(k, grid, dim3(256), 0, s, q, rpw, strips);                                    \
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, s, q, rpw, strips, ls);                           \
     return;                                                                                     \
   }
   P0_STAGE(P0_XMODE_F16)

@@ -213,10 +213,11 @@ def test_gemm_flux_shape_sampled_rows(dev):
 
 
 @pytest.mark.parametrize("mode", ["f16", "bf16", "lnmod", "rms"])
-@pytest.mark.parametrize("M,K,pad", [(3, 544, 0), (9001, 32, 0), (33005, 32, 0), (2051, 2592, 1)])
+@pytest.mark.parametrize("M,K,pad", [(3, 544, 0), (9001, 32, 0), (33005, 32, 0), (2051, 2592, 1), (131077, 32, 0),
+                                     (700, 96, 1), (8200, 544, 0), (2100, 512, 1)])
 def test_gemm_staging_rows_per_wave(dev, mode, M, K, pad):
-    """the activation staging where a wave walks 1, 4 and 8 rows (3, 9001 and 33005 x one strip; 2051 x six, the last of
-    32 columns), with a ragged last row group, 16-byte aligned rows and rows that are not (a leading element). One fp32
+    """the activation staging where a wave walks 1, 4 and 8 steps, a step 1 to 16 rows side by side (as many lanes a row as K
+    fills), with a ragged last step and row group, 16-byte aligned rows and rows that are not (a leading element). One fp32
     rounding may differ from the oracle's before the value is rounded to fp16, which flips about 2^-12 of the fp16
     roundings by 2^-11: 1.3e-5 relative; the bar is four times that"""
     N, ld, c0 = 64, K + 8 * pad, pad if mode != "f16" else 1
