@@ -442,8 +442,9 @@ static int slices(const GemmP& p, int64_t tiles, int steps) {
 static int64_t tiles_of(const GemmP& p, int bm, int bn) { return ((int64_t)p.N + bn - 1) / bn * (((int64_t)p.M + bm - 1) / bm); }
 
 // Forms: whole 64-row weight tiles (the first weight rows multiples of 64), records 16-byte aligned, X' rows and the weight
-// within 32-bit offsets (unsigned ones: rows that go down in memory stay on gemm.hip, which adds 64-bit offsets). Then by time: a step of 64 k takes this kernel 1.0 us a round of 256 workgroups and about 4 us a
-// call, 12 with K slices (the partials); the 256 x 256 tiles of gemm.hip 1.4 us while one round holds them all, and 9 us.
+// within 32-bit offsets (unsigned ones: rows that go down in memory stay on gemm.hip, which adds 64-bit offsets). Then by
+// time: a step of 64 k takes this kernel 1.0 us a round of 256 workgroups, 1.2 us a round, and about 3 us a call, 11 with K
+// slices (the partials); the 256 x 256 tiles of gemm.hip 1.4 us while one round holds them all, and 9 us.
 // Measured (us, this kernel / gemm.hip): M = 256: 3072 x 2048 21 / 55, 16384 x 2048 swiglu 36 / 62, 2048 x 8192 33 / 179;
 // M = 512: 3072 x 3072 35 / 77, 3072 x 9216 75 / 205, 9216 x 3072 95 / 82; M = 1024: 3072 x 9216 128 / 210; M = 2048:
 // 3072 x 3072 93 / 82.
@@ -454,7 +455,8 @@ bool n128_takes(const GemmP& p) {
   const int steps = (p.K + 63) / 64;
   const int64_t small = tiles_of(p, Tile::BMt, Tile::BNt), big = tiles_of(p, 256, 256);
   const int nks = slices(p, small, steps);
-  const int64_t here = (small * nks + 255) / 256 * ((steps + nks - 1) / nks) * 10 + (nks > 1 ? 120 : 40);   // 0.1 us
+  const int64_t rounds = (small * nks + 255) / 256;
+  const int64_t here = rounds * ((steps + nks - 1) / nks * 10 + 12) + (nks > 1 ? 108 : 28);   // 0.1 us
   return here < (big + 255) / 256 * steps * 14 + 90;
 }
 
