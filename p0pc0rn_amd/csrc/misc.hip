@@ -345,9 +345,10 @@ __global__ __launch_bounds__(kNaThreads) void normadd_few_kernel(const float* __
 }
 
 // engine/llm/lops.js:418-433, engine/llm/lops_spec.js:329-343: (value, index) with ties to the lower index. A running
-// best is never NaN, so "better" is a total order on what is combined: any order of the reduction gives its result. One
-// workgroup per row, four pairs in flight per thread: 16 waves for a head's 4096 tile maxima in one round (256 threads that
-// loaded 16 pairs one after another took 6.3 us a launch, this 4.0), 4 for shorter rows, or many of them.
+// best is never NaN, so "better" is a total order on what is combined: any order of the reduction gives its result. A
+// workgroup of 16 waves per row, four pairs in flight per thread: a head's 4096 tile maxima in one round, 4.0 us a launch (256
+// threads that load 16 pairs one after another: 6.3).
+constexpr int kArgThreads = 1024;
 typedef uint32_t u32x2a4 __attribute__((ext_vector_type(2), aligned(4)));   // an 8-byte load at 4-byte alignment
 __device__ __forceinline__ bool better(float v, uint32_t id, float bv, uint32_t bi) {
   return v > bv || (v == bv && id < bi);
@@ -360,7 +361,6 @@ __device__ __forceinline__ void wave_best(float& v, uint32_t& id) {
     if (better(ov, oi, v, id)) { v = ov; id = oi; }
   }
 }
-template <int kArgThreads>
 __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const float* __restrict__ MX, int64_t n,
                                                             uint32_t* __restrict__ out) {
   __shared__ float rv[kArgThreads / 64];
@@ -395,6 +395,33 @@ __global__ __launch_bounds__(kArgThreads) void argmax_kernel(const float* __rest
   if (lane == 0) {
     out[2 * blockIdx.x] = bi;
     out[2 * blockIdx.x + 1] = __float_as_uint(bv);
+  }
+}
+
+// The same with 256 threads, one pair at a time, and a tree through LDS: short rows, or many.
+__global__ __launch_bounds__(kRowThreads) void argmax_short_kernel(const float* __restrict__ MX, int64_t n,
+                                                                   uint32_t* __restrict__ out) {
+  __shared__ float rv[kRowThreads];
+  __shared__ uint32_t ri[kRowThreads];
+  const int t = threadIdx.x;
+  const int64_t b = (int64_t)blockIdx.x * n;
+  float bv = -3.4e38f;
+  uint32_t bi = 0xFFFFFFFFu;
+  for (int64_t i = t; i < n; i += kRowThreads) {
+    const float v = MX[2 * (b + i)];
+    const uint32_t id = __float_as_uint(MX[2 * (b + i) + 1]);
+    if (better(v, id, bv, bi)) { bv = v; bi = id; }
+  }
+  rv[t] = bv;
+  ri[t] = bi;
+  __syncthreads();
+  for (int s = kRowThreads / 2; s > 0; s >>= 1) {
+    if (t < s && better(rv[t + s], ri[t + s], rv[t], ri[t])) { rv[t] = rv[t + s]; ri[t] = ri[t + s]; }
+    __syncthreads();
+  }
+  if (t == 0) {
+    out[2 * blockIdx.x] = ri[0];
+    out[2 * blockIdx.x + 1] = __float_as_uint(rv[0]);
   }
 }
 
@@ -493,12 +520,11 @@ extern "C" int p0_argmaxM(const float* mx, int64_t n, int64_t M, uint32_t* out) 
   if (n < 0 || M < 1) { set_error("argmax: n %lld, M %lld", (long long)n, (long long)M); return P0_EINVAL; }
   if (int r = require_open("argmax")) return r;
   if (building_chain()) return chain_add_argmax(mx, n, M, out);
-  // 16 waves pay where one row's pairs are worth them and the rows do not fill the chip by themselves (us, 4 waves that loaded
-  // one pair at a time / 16: one row of 256 pairs 2.8 / 3.1, of 1536 3.5 / 3.2, 512 rows of 2048 4.1 / 4.3, of 3072 4.7 / 4.3,
-  // 2048 rows of 256 3.6 / 9.3)
+  // 16 waves pay where one row's pairs are worth them and the rows do not fill the chip by themselves (us, 4 waves / 16: one row
+  // of 256 pairs 2.8 / 3.1, of 1536 3.5 / 3.2, 512 rows of 2048 4.1 / 4.3, of 3072 4.7 / 4.3, 2048 rows of 256 3.6 / 9.3)
   const bool wide = n > 1024 && n >= 6 * M;
-  auto k = wide ? argmax_kernel<1024> : argmax_kernel<256>;
-  hipLaunchKernelGGL(k, dim3((unsigned)M), dim3(wide ? 1024 : 256), 0, ctx().cur, mx, n, out);
+  auto k = wide ? argmax_kernel : argmax_short_kernel;
+  hipLaunchKernelGGL(k, dim3((unsigned)M), dim3(wide ? kArgThreads : kRowThreads), 0, ctx().cur, mx, n, out);
   P0_LAUNCHED("argmax");
   return P0_OK;
 }
