@@ -45,7 +45,7 @@ __device__ __forceinline__ int swz(int r, int c) { return r * 128 + ((c ^ swz_ke
 
 // ------------------------------------------------------------------------------------------------ X staging
 // Bound: HBM, one read of X and one write of X'. A wave owns a strip of 8 L columns (8 per lane: a 16-byte store, one or
-// two 16-byte loads; L = 1 << ls lanes a row, 64 unless that would leave more than an eighth of them past K) of 64 / L rows
+// two 16-byte loads; L = 1 << ls lanes a row, 64 unless that would leave nearly as many past K as before it) of 64 / L rows
 // side by side and walks `rpw` such steps down it, UR steps' loads in flight, so that the modulation vectors of an lnmod
 // are loaded once per strip and no index is divided. 4608 x 3072, lnmod: 59 -> 14.5 us, 5.9 TB/s (one chunk of 8 per thread
 // with a 64-bit division and 16 scalar modulation loads each, before). With 64 lanes a row always, the calls of 65536 rows
@@ -123,14 +123,17 @@ __global__ __launch_bounds__(256) void x_stage_kernel(XStageP p, int rpw, int st
   }
 }
 
-// steps a wave walks: one while that gives the chip no more than 8 waves per SIMD (8192 in all), up to 8 beyond
+// steps a wave walks. One while that gives the chip no more than 8 waves per SIMD (8192 in all). Beyond, up to 8 where they
+// share an lnmod's vectors, or where a strip is the whole row (whole GEMM, bf16, 1 step / 8: 65536 x 128 32.9 / 28.9 us, 32768
+// x 256 24.8 / 20.1), else one (16384 x 3072 65.3 / 66.5, 65536 x 544 52.7 / 53.8)
 static void launch_x_stage(const XStageP& q, hipStream_t s) {
-  const int chunks = q.K / 8;   // a multiple of 4
+  const int chunks = q.K / 8;   // a multiple of 4: 4 lanes always fit
   int ls = 6;
-  while (((chunks + (1 << ls) - 1) >> ls << ls) - chunks > chunks / 8) --ls;   // 4 lanes always fit
+  while (5 * (((chunks + (1 << ls) - 1) >> ls << ls) - chunks) > 4 * chunks) --ls;
   const int strips = (chunks + (1 << ls) - 1) >> ls, side = 64 >> ls;
   const int64_t steps = ((int64_t)q.M + side - 1) / side, waves = (int64_t)strips * steps;
-  int rpw = waves <= 8192 ? 1 : waves <= 32768 ? 4 : 8;
+  const bool f32 = q.xmode == P0_XMODE_LNMOD || q.xmode == P0_XMODE_RMS;
+  int rpw = waves <= 8192 ? 1 : strips == 1 ? 8 : !f32 ? 1 : waves <= 32768 ? 4 : 8;
   while (waves / rpw > (1 << 25)) rpw *= 2;   // a grid of at most 2^32 threads
   const dim3 grid((unsigned)((steps + 4 * rpw - 1) / (4 * rpw) * strips));
 #define P0_STAGE(MODE)                                                                          \
