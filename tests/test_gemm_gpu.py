@@ -303,3 +303,51 @@ def test_gemm_rows_going_down_in_memory(dev, M, mode):
     check(got, want, f"gemm {mode} rows down {M}x{N}x{K}", 1e-5)
     up, _ = run(dict(f, x_ld=ld), dict(w=w, x=np.ascontiguousarray(x.reshape(M, ld)[::-1])), np.float32, M * N)
     assert np.array_equal(up.view(np.uint32), want.view(np.uint32))
+
+
+def _hard_records(N, K, seed):
+    """q4 records a third of whose (row, group) pairs have q s + m inexact in fp32: a scale far above its minimum (odd
+    mantissas, so that 3 s, 6 s and 12 s lie half way between fp16 values and the minimum decides), a minimum far above its
+    scale, subnormals of either"""
+    rng = np.random.default_rng(seed)
+    w = O.pack_q4(O.randn(N * K, seed, 0.05), N, K)[0].copy().view(np.uint32).reshape(N // 64, K // 32, 320)
+    w[..., :256] = rng.integers(0, 1 << 32, w[..., :256].shape, dtype=np.uint32)
+    sm = w[..., 256:].copy().view(np.float16).reshape(N // 64, K // 32, 64, 2)
+    kind = rng.integers(0, 9, sm.shape[:3])
+    odd = (rng.integers(512, 682, sm.shape[:3]) * 2 + 1) / 1024.0
+    e = rng.integers(2, 9, sm.shape[:3]).astype(np.float64)
+    sign = rng.choice([-1.0, 1.0], sm.shape[:3])
+    s = np.select([kind == 0, kind == 1, kind == 2], [odd * 2.0 ** e, odd * 2.0 ** (e - 14), odd * 2.0 ** -16], sm[..., 0])
+    m = np.select([kind == 0, kind == 1, kind == 2], [sign * odd * 2.0 ** (e - 25), sign * odd * 2.0 ** e, sign * odd], sm[..., 1])
+    sm[..., 0], sm[..., 1] = s.astype(np.float16), m.astype(np.float16)
+    w[..., 256:] = sm.reshape(N // 64, K // 32, 128).view(np.uint32)
+    return w.reshape(-1).view(np.uint8), sm
+
+
+def test_gemm_weights_that_round_twice(dev):
+    """each weight is fl16(fl32(q s + m)), bit for bit, also where the one rounding of the packed fp16 path would differ: rows
+    of X that pick one k each give the weights themselves, in 128 x 128 tiles with K slices and a last step of one group, and
+    in 256 x 256 tiles (the weight at a 4-byte offset)"""
+    M, N, K = 200, 192, 2080
+    w, sm = _hard_records(N, K, 5)
+    w16 = np.asarray(O.dequant_q4(w, N, K)[1]).view(np.float16)
+    q = w.view(np.uint32).reshape(N // 64, K // 32, 320)[..., :256].reshape(N // 64, K // 32, 64, 4)
+    q = ((q[..., None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(N // 64, K // 32, 64, 32)
+    one = (q * sm[..., :1].astype(np.float64) + sm[..., 1:].astype(np.float64)).astype(np.float16)   # exact, rounded once
+    one = one.transpose(0, 2, 1, 3).reshape(N, K)
+    differ = (one.view(np.uint16) != w16.view(np.uint16)).sum(0)
+    ks = np.concatenate([np.argsort(-differ)[:M - 40], np.arange(K - 40, K)])   # the columns with most of them, and the tail
+    print("weights that round twice among those compared:", int(differ[ks].sum()), flush=True)
+    assert differ[ks].sum() > 500
+    x = np.zeros((M, K), np.float16)
+    x[np.arange(M), ks] = 1
+    f = dict(w_rows=N, w_cols=K, M=M, N=N, K=K, x_mode=capi.XMODE["f16"], epi=capi.GEPI["f32"])
+    want = np.ascontiguousarray(w16[:, ks].T.astype(np.float32))
+    for off in (0, 4):
+        wb = capi.to_device(np.concatenate([np.zeros(off, np.uint8), w]))
+        xb, yb = capi.to_device(x), capi.Buffer(want.nbytes).fill_u32(NAN32)
+        capi.q4_gemm(capi.gemm_args(**f, w=wb, w_off=off, x=xb, y=yb))
+        got = yb.read(np.float32).reshape(M, N)
+        assert np.array_equal(got, want), f"weight offset {off}: {int((got != want).sum())} differ"
+        for b in (wb, xb, yb):
+            b.free()
