@@ -163,9 +163,11 @@ def test_gemv_deterministic(dev):
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-def test_gemv_decompositions_agree(dev):
-    """the split-K decomposition is a tuning choice: every choice gives the oracle's result"""
-    c = Case(1, 1024, 4096, "raw", "store", kPer=2048, seed=17)
+@pytest.mark.parametrize("K,kPer", [(2816, 0), (4096, 2048)])
+def test_gemv_decompositions_agree(dev, K, kPer):
+    """the split-K decomposition of gemv.hip (one split of more than 2048 k) is a tuning choice: every choice gives the
+    oracle's result. Splits of 2048 k run on gemv1.hip, whatever the knobs say"""
+    c = Case(1, 1024, K, "raw", "store", kPer=kPer, seed=17)
     want = c.run_oracle()[0]
     idx = c.rows_written()
     old = [capi.gemv_tune(k) for k in range(4)]
@@ -180,15 +182,17 @@ def test_gemv_decompositions_agree(dev):
             capi.gemv_tune(k, v)
 
 
-def test_gemv_split_k_workspace_across_reopen(dev):
-    """K in many slices per workgroup (the uncached split-K workspace and its arrival counters), run after run, then
-    after closing and reopening the device (the workspace is kept, not freed): the same bits, the oracle's values"""
-    c = Case(1, 512, 4096, "rms", "store", kPer=2048, seed=23)
+@pytest.mark.parametrize("M,K,kPer", [(1, 2816, 0), (1, 4096, 2048), (5, 16384, 0)])
+def test_gemv_split_k_workspace_across_reopen(dev, M, K, kPer):
+    """K in many slices over workgroups (the uncached split-K workspace and its arrival counters: gemv.hip's, and gemvm.hip's
+    for a long split), run after run, then after closing and reopening the device (the workspace is kept, not freed): the
+    same bits, the oracle's values. Splits of 2048 k at M = 1 keep K in the workgroup (gemv1.hip)"""
+    c = Case(M, 512, K, "rms", "store", kPer=kPer, seed=23, gemvM=M > 1)
     want = c.run_oracle()[0]
     idx = c.rows_written()
     old = [capi.gemv_tune(k) for k in range(4)]
     try:
-        for k, v in enumerate((100000, 100000, 1, 2)):   # 2 waves per slot, 1 group per wave: 32 slices per split
+        for k, v in enumerate((100000, 100000, 1, 2)):   # gemv.hip: 2 waves per slot, 1 group per wave, 44 slices
             capi.gemv_tune(k, v)
         runs = [c.run_gpu()[0] for _ in range(3)]
         capi.close_device()
@@ -203,16 +207,17 @@ def test_gemv_split_k_workspace_across_reopen(dev):
 
 
 @pytest.mark.parametrize("M,epi,K,kPer", [(3, "store", 4096, 2048), (5, "geglu", 2048, 0), (16, "store", 4096, 2048),
-                                          (4, "store", 3168, 1024), (1, "store", 3168, 1024)])
+                                          (4, "store", 3168, 1024), (1, "store", 3168, 1024), (1, "store", 2976, 0),
+                                          (1, "softcap", 2848, 0)])
 def test_gemvM_many_k_slices(dev, M, epi, K, kPer):
-    """gemvM (matrix cores) with K in many slices: the last workgroup to arrive loads the slices' partials of every x
-    row in batches (fewer slices per batch as M grows) and adds them in slice order; the oracle's values. K = 3168 in
-    splits of 1024 leaves a last split of 3 groups, whose later slices hold no group (they store zeros and still count
-    their arrival); at M = 1 the same through gemv"""
+    """gemv.hip's kernel with K in many slices (knob 4 keeps M > 1 there): the last workgroup to arrive loads the slices'
+    partials of every x row in batches (fewer slices per batch as M grows) and adds them in slice order; the oracle's
+    values. K = 3168 in splits of 1024 leaves a last split of 3 groups, whose later slices hold no group (they store zeros
+    and still count their arrival). At M = 1 one split of more than 2048 k, 93 and 89 groups in slices of 2, the last of one"""
     c = Case(M, 256, K, "rms", epi, kPer=kPer, seed=29 + M, gemvM=M > 1)
-    old = [capi.gemv_tune(k) for k in range(4)]
+    old = [capi.gemv_tune(k) for k in range(5)]
     try:
-        for k, v in enumerate((100000, 100000, 1, 2)):
+        for k, v in enumerate((100000, 100000, 1, 2, 17)):
             capi.gemv_tune(k, v)
         c.check(f"gemvM M={M} {epi}, many K slices")
     finally:
@@ -296,9 +301,9 @@ def test_gemvM_two_tiles_per_wave(dev, mf):
 
 @pytest.mark.parametrize("M", [2, 5, 16])
 def test_gemvM_large_activations_keep_fp32(dev, mf, M):
-    """M >= 2 runs on MFMA with 2^8 x' split into fp16 hi + lo; a workgroup whose x' reaches 255 (fp16 would
-    overflow) takes the fp32 path instead. Large values sit in one K-slice only, so both paths run in one call, and the
-    split partials still meet the fp32 bar."""
+    """x rows with values far above the others in one split, the fp32 bar in every split: on the VALU x' stays fp32; on the
+    matrix cores it is split into fp16 hi + lo under a scale of its own per row and wave, so that large values neither
+    overflow nor take the others' bits"""
     c = Case(M, 128, 8192, "raw", "store", kPer=2048, seed=62 + M, gemvM=True)
     for m in range(M):
         c.x[m * 8192 + 4096: m * 8192 + 4096 + 7] = np.float32([400.0, -900.0, 330.0, 1.0e5, -3.5e3, 600.0, 2.0e4])
