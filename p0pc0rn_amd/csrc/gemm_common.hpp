@@ -76,7 +76,10 @@ __device__ __forceinline__ u32x4n deq_word(uint32_t v, uint32_t sm, bool fast) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float q0 = (float)((v >> (8 * j)) & 15u), q1 = (float)((v >> (8 * j + 4)) & 15u);
-      o[j] = pack_h2(__builtin_fmaf(q0, s, m), __builtin_fmaf(q1, s, m));
+      // two roundings: left to itself, the compiler folds the fma and the conversion into one v_fma_mixlo_f16, which rounds once
+      float f0 = __builtin_fmaf(q0, s, m), f1 = __builtin_fmaf(q1, s, m);
+      asm("" : "+v"(f0), "+v"(f1));
+      o[j] = pack_h2(f0, f1);
     }
   }
   return o;

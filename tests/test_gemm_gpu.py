@@ -345,9 +345,11 @@ def test_gemm_weights_that_round_twice(dev):
     want = np.ascontiguousarray(w16[:, ks].T.astype(np.float32))
     for off in (0, 4):
         wb = capi.to_device(np.concatenate([np.zeros(off, np.uint8), w]))
-        xb, yb = capi.to_device(x), capi.Buffer(want.nbytes).fill_u32(NAN32)
+        xb, yb, hb = capi.to_device(x), capi.Buffer(want.nbytes).fill_u32(NAN32), capi.Buffer(2 * N * K)
+        capi.q4_dequant(wb, N, K, out16=hb, w_off=off)
+        assert np.array_equal(hb.read(np.uint16), w16.view(np.uint16).ravel())
         capi.q4_gemm(capi.gemm_args(**f, w=wb, w_off=off, x=xb, y=yb))
         got = yb.read(np.float32).reshape(M, N)
         assert np.array_equal(got, want), f"weight offset {off}: {int((got != want).sum())} differ"
-        for b in (wb, xb, yb):
+        for b in (wb, xb, yb, hb):
             b.free()
