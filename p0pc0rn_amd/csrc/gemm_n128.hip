@@ -140,23 +140,14 @@ __global__ __launch_bounds__(64 * WM * WN) void n128_kernel(N128P a) {
     dma16(d + C::CBytes + (wv % C::SL) * 1024, sv + (one ? 0 : sg * 1280), rs, sc * 2560);
   };
   // ---- dequant of step st's records into W tile st & 1: thread -> slot tid % BNt, words WPT (tid / BNt) .. of its 8
-  const int dslot = tid % C::BNt, dw = tid / C::BNt * C::WPT, dg = dw >> 2;   // WPT <= 4: one group
+  const int dslot = tid % C::BNt, dw = tid / C::BNt * C::WPT, dg = dw >> 2;   // two words: one group
   const int dkey = key(dslot);
   uint32_t w[C::WPT], sm;
   auto read_raw = [&](int st) {
     const uint8_t* rw = lds + S * C::XBytes + (st % S) * C::RBytes;
-    const uint32_t* cw = (const uint32_t*)(rw + dg * (C::BNt * 16) + dslot * 16 + (dw & 3) * 4);
-    if constexpr (C::WPT == 4) {
-      const u32x4n v = *(const u32x4n*)cw;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) w[i] = v[i];
-    } else if constexpr (C::WPT == 2) {
-      const uint2 v = *(const uint2*)cw;
-      w[0] = v.x;
-      w[1] = v.y;
-    } else {
-      w[0] = *cw;
-    }
+    const uint2 v = *(const uint2*)(rw + dg * (C::BNt * 16) + dslot * 16 + (dw & 3) * 4);
+    w[0] = v.x;
+    w[1] = v.y;
     sm = *(const uint32_t*)(rw + C::CBytes + dg * (C::BNt * 4) + dslot * 4);
   };
   auto write_w = [&](int st, const u32x4n (&d)[C::WPT]) {
@@ -172,7 +163,7 @@ __global__ __launch_bounds__(64 * WM * WN) void n128_kernel(N128P a) {
       if (!pk_exact(sm)) write_w(st, d);
     }
   };
-  static_assert(C::WPT == 1 || C::WPT == 2 || C::WPT == 4, "whole words of one group per thread");
+  static_assert(C::WPT == 2, "two code words of one group per thread");
 
   const int hh = lane >> 5, frow = lane & 31, fkey = key(frow);
   u32x4n av[2][2], bv[2][NT];
@@ -433,7 +424,7 @@ int n128_init() {
 }
 
 // K slices: as many as keep one workgroup per CU, each of at least 8 steps, partials within the workspace
-static int slices(const GemmP& p, int64_t tiles, int steps) {
+static int slices(int64_t tiles, int steps) {
   int nks = (int)(256 / tiles);
   if (nks > steps / 8) nks = steps / 8;
   while (nks > 1 && (size_t)tiles * nks * Tile::BMt * Tile::BNt > ctx().part_floats) --nks;
@@ -454,7 +445,7 @@ bool n128_takes(const GemmP& p) {
   if (p.ldx < 0 || p.ldx >= (1 << 21) || (p.Nw >> 6) * p.wG * 1280 >= (1ll << 31)) return false;
   const int steps = (p.K + 63) / 64;
   const int64_t small = tiles_of(p, Tile::BMt, Tile::BNt), big = tiles_of(p, 256, 256);
-  const int nks = slices(p, small, steps);
+  const int nks = slices(small, steps);
   const int64_t rounds = (small * nks + 255) / 256;
   const int64_t here = rounds * ((steps + nks - 1) / nks * 10 + 12) + (nks > 1 ? 108 : 28);   // 0.1 us
   return here < (big + 255) / 256 * steps * 14 + 90;
@@ -465,7 +456,8 @@ void launch_n128(const GemmP& p, hipStream_t s) {
   a.g = p;
   const int steps = (p.K + 63) / 64;
   const int64_t tiles = tiles_of(p, Tile::BMt, Tile::BNt);
-  a.spk = (steps + slices(p, tiles, steps) - 1) / slices(p, tiles, steps);
+  const int nks = slices(tiles, steps);
+  a.spk = (steps + nks - 1) / nks;
   a.nks = (steps + a.spk - 1) / a.spk;
   a.part = ctx().part;
   a.cnt = ctx().gemm_counters;   // one per tile where there are slices: at most 128 tiles

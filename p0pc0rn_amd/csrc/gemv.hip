@@ -59,13 +59,13 @@ static Plan plan(int M, int NT, int epi, int nsplit, int kPer) {
   pl.rowsTot = (epi == P0_EPI_GEGLU ? 2 : 1) * NT * 64;
   const int Gs = kPer / 32;
   // K shares per slot and split: enough waves for the chip, but at least g_min_gpw groups each. A geglu slot streams
-  // the gate and the up tile and counts twice at M = 1 and from M = 12 on; at M = 2-8 the extra K-slices' partials cost
-  // more than the parallelism gains (measured on the E2B gate_up: 14-20 us per launch against 20-26)
+  // the gate and the up tile and counts twice at M = 1 and from M = 12 on (p0_gemv_tune knob 4 = 17; 2 x 8192 x 2048, 12 and
+  // 16 rows: 40 and 49 us per launch against 48 and 63); in between the extra K-slices' partials cost more than they give
   const int work = pl.mode == 2 && (M == 1 || M >= 12) ? 2 * g_target_waves : g_target_waves;
   int kws = (work + slots * nsplit - 1) / (slots * nsplit);
-  // 12-16 x rows over several kPer splits (the E2B down projection): the splits already give the chip its workgroups,
-  // and K-slices would multiply the partials of every row; two waves per slot, K in one workgroup per split
-  // (measured at M = 12 / 16: 25-26 us per launch against 31-32)
+  // 12-16 x rows over several kPer splits (knob 4 = 17): the splits already give the chip its workgroups, and K-slices would
+  // multiply the partials of every row; two waves per slot, K in one workgroup per split (16 rows, 2560 x 10240 in 5 splits: 54
+  // us against 61; 2048 x 8192 in 4: 45 against 42)
   if (M >= 12 && nsplit >= 4 && kws > 2) kws = 2;
   const int kws_max = Gs / g_min_gpw > 1 ? Gs / g_min_gpw : 1;
   if (kws > kws_max) kws = kws_max;
