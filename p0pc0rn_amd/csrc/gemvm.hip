@@ -49,10 +49,18 @@ __device__ __forceinline__ half8_t codes_q8(uint32_t w0, uint32_t w1) {
   return __builtin_bit_cast(half8_t, u);
 }
 
+// The arguments of a launch in K slices (on their own: 24 bytes more for every launch cost the others 1%)
+struct GmSliceP : GmP {
+  int nks, pps;                // K slices per split, over workgroups, and the passes of a slice
+  float* part; unsigned* cnt;  // the slices' sums and the arrival counts (the split-K workspace)
+};
+template <bool SLICED> struct GmArgs { typedef GmP type; };
+template <> struct GmArgs<true> { typedef GmSliceP type; };
+
 // One launch: grid (workgroups, splits x K slices); workgroup pos takes items [pos ipw, (pos + 1) ipw) of its split. SLICED:
 // p.nks > 1 slices of a split, one item per workgroup
 template <int ENC, int NBK, bool GEGLU, bool PLEG, bool SLICED>
-__global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
+__global__ __launch_bounds__(kGmThreads) void gemvm_kernel(typename GmArgs<SLICED>::type p) {
   constexpr bool Q4 = ENC == P0_ENC_Q4G32A_T64;
   constexpr int GK = Q4 ? 32 : 64;             // k per group
   constexpr int RJ = Q4 ? 2 : 4;               // record loads per block and pass: quads of groups (q4), groups (q8)
@@ -64,13 +72,20 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int M = p.M, l16 = lane & 15, q = lane >> 4, m = min(l16, M - 1);
   const int pos = stage_pos(blockIdx.x, p.wgs);
-  const int split = SLICED ? (int)blockIdx.y / p.nks : blockIdx.y, ks = SLICED ? (int)blockIdx.y - split * p.nks : 0;
+  int split = blockIdx.y, ks = 0;
+  if constexpr (SLICED) {
+    split = (int)blockIdx.y / p.nks;
+    ks = (int)blockIdx.y - split * p.nks;
+  }
   const int it0 = pos * p.ipw, it1 = min(p.items, it0 + p.ipw);
   if (it0 >= it1) return;
   // the workgroup's k: its split, or its slice of it (none, for the last slices of a last split shorter than the others)
-  const int k0s = split * p.kPer + ks * p.pps * kGmPass;
-  const int k1s = SLICED ? min(min(p.K, (split + 1) * p.kPer), k0s + p.pps * kGmPass) : min(p.K, k0s + p.kPer);
-  const int passes = SLICED ? max(0, (k1s - k0s + kGmPass - 1) / kGmPass) : (k1s - k0s + kGmPass - 1) / kGmPass;
+  int k0s = split * p.kPer, k1s = min(p.K, k0s + p.kPer);
+  if constexpr (SLICED) {
+    k0s += ks * p.pps * kGmPass;
+    k1s = max(k0s, min(k1s, k0s + p.pps * kGmPass));
+  }
+  const int passes = (k1s - k0s + kGmPass - 1) / kGmPass;
 
   // weight row of block b of item it (a geglu's blocks U .. NBK - 1: the up rows)
   auto block_row = [&](int it, int b) { return (it * U + (GEGLU ? b % U : b)) * 16 + (GEGLU && b >= U ? p.N : 0); };
@@ -115,7 +130,10 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   constexpr int RUN = 256 / RJ, CR = 8 / RJ;
   const int kq = Q4 ? 8 * q : 16 * q;
   auto kl = [](int c) { return Q4 ? (c % CR) * 32 : 8 * (c % CR); };
-  auto at_k = [&](int c, int ng) { return in_pass(c, ng) ? (wv + kGmWaves * (c / CR)) * RUN + kl(c) : 0; };   // uniform
+  // the k a chunk's loads take (uniform): past the split the wave's first chunk again, whose x' set no other scale for the row
+  auto at_k = [&](int c, int ng) {
+    return in_pass(c, ng) ? (wv + kGmWaves * (c / CR)) * RUN + kl(c) : in_pass(0, ng) ? wv * RUN : 0;
+  };
   u32x4 xv[8][2], nv;
   float rstd = 1.0f;
   const bool rms = p.pro == P0_PRO_RMS;
@@ -182,7 +200,7 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
           if (m >= r0 && m < r0 + 4)
 #pragma unroll
             for (int c = 0; c < 8; ++c) {
-              const float* xr = nws[wv] + (m - r0) * kPlegRow + (c / CR) * RUN + kl(c) + kq;
+              const float* xr = nws[wv] + (m - r0) * kPlegRow + (in_pass(c, ng) ? (c / CR) * RUN + kl(c) : 0) + kq;
               const float4 x0 = *(const float4*)xr, x1 = *(const float4*)(xr + 4);
               v[c][0] = x0.x; v[c][1] = x0.y; v[c][2] = x0.z; v[c][3] = x0.w;
               v[c][4] = x1.x; v[c][5] = x1.y; v[c][6] = x1.z; v[c][7] = x1.w;
@@ -224,7 +242,7 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[c][e] = __uint_as_float(xv[c][e >> 2][e & 3]);
         if (rms) {
-          const float* nr = nws[wv] + (c / CR) * RUN + kl(c) + kq;
+          const float* nr = nws[wv] + (in_pass(c, ng) ? (c / CR) * RUN + kl(c) : 0) + kq;   // as at_k
           const float4 n0 = *(const float4*)nr, n1 = *(const float4*)(nr + 4);
           const float n[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
 #pragma unroll
@@ -233,13 +251,12 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
       }
     }
     // the row's largest |x'| over the wave's k (the lanes of a row are 16 apart): an infinity makes it infinite, a NaN
-    // stays out of it, and so does what the loads of a chunk past the split returned (other k, other norm weights)
+    // stays out of it
     float big = 0.0f;
 #pragma unroll
     for (int c = 0; c < 8; ++c)
-      if (in_pass(c, ng))
 #pragma unroll
-        for (int e = 0; e < 8; e += 2) big = fmaxf(fmaxf(big, __builtin_fabsf(v[c][e])), __builtin_fabsf(v[c][e + 1]));
+      for (int e = 0; e < 8; e += 2) big = fmaxf(fmaxf(big, __builtin_fabsf(v[c][e])), __builtin_fabsf(v[c][e + 1]));
     auto over_row = [](float b) {
       const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(b), __float_as_uint(b), false, false);
       b = fmaxf(__uint_as_float(s[0]), __uint_as_float(s[1]));
@@ -252,12 +269,11 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
       big = 0.0f;
 #pragma unroll
       for (int c = 0; c < 8; ++c)
-        if (in_pass(c, ng))
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float a = __builtin_fabsf(v[c][e]);
-            big = fmaxf(big, a < __builtin_inff() ? a : 0.0f);
-          }
+        for (int e = 0; e < 8; ++e) {
+          const float a = __builtin_fabsf(v[c][e]);
+          big = fmaxf(big, a < __builtin_inff() ? a : 0.0f);
+        }
       big = over_row(big);
     }
     const int ex = (int)((__float_as_uint(big) >> 23) & 255u) - 127;   // floor(log2 big); -127 for 0 and subnormals
@@ -343,8 +359,10 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
   };
 
   // where slice s of this workgroup's item keeps the sum of x row mm, row l16 of block b (h = 1: a geglu's up row)
-  auto slice_at = [&](int s, int mm, int b, int h) {
-    return p.part + ((((int64_t)(split * p.items + it0) * p.nks + s) * (GEGLU ? 2 : 1) + h) * M * U + mm * U + b) * 16 + l16;
+  auto slice_at = [&](int s, int mm, int b, int h) -> float* {
+    if constexpr (SLICED)
+      return p.part + ((((int64_t)(split * p.items + it0) * p.nks + s) * (GEGLU ? 2 : 1) + h) * M * U + mm * U + b) * 16 + l16;
+    return nullptr;
   };
   auto slice_store = [&](int mm, int b, float v0, float v1) {
     stf<true>(slice_at(ks, mm, b, 0), v0);
@@ -391,66 +409,68 @@ __global__ __launch_bounds__(kGmThreads) void gemvm_kernel(GmP p) {
       else epilogue<false>(p, split, mm, n >> 6, n & 63, v0, v1);
     }
   }
-  if constexpr (!SLICED) return;
-  // the last of an item's slices to arrive adds their sums in slice order. The workspace
-  // is uncached memory: a store is in memory once acknowledged, so the arrival count needs no fence
-  __shared__ int s_last;
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  if (tid == 0) {
-    auto* c = P0_GLOBAL(unsigned, p.cnt + split * p.items + it0);
-    s_last = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(p.nks - 1);
-    if (s_last) __hip_atomic_exchange(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // leave it at zero
-  }
-  __syncthreads();
-  if (!s_last) return;
-  for (int r = tid >> 4; r < M * U; r += kGmThreads / 16) {
-    const int mm = r / U, b = r - mm * U, n = (it0 * U + b) * 16 + l16;
-    float v[2] = {0.0f, 0.0f};
-    for (int s0 = 0; s0 < p.nks; s0 += 8) {   // 8 slices in flight; past the last: the last again, not added
-      float t[8][GEGLU ? 2 : 1];
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-#pragma unroll
-        for (int h = 0; h < (GEGLU ? 2 : 1); ++h) t[u][h] = ldf<true>(slice_at(min(s0 + u, p.nks - 1), mm, b, h));
-#pragma unroll
-      for (int u = 0; u < 8; ++u)
-        if (s0 + u < p.nks)
-#pragma unroll
-          for (int h = 0; h < (GEGLU ? 2 : 1); ++h) v[h] += t[u][h];
+  if constexpr (SLICED) {
+    // the last of an item's slices to arrive adds their sums in slice order. The workspace
+    // is uncached memory: a store is in memory once acknowledged, so the arrival count needs no fence
+    __shared__ int s_last;
+    __builtin_amdgcn_s_waitcnt(0);
+    __syncthreads();
+    if (tid == 0) {
+      auto* c = P0_GLOBAL(unsigned, p.cnt + split * p.items + it0);
+      s_last = __hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)(p.nks - 1);
+      if (s_last) __hip_atomic_exchange(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // leave it at zero
     }
-    epilogue<false>(p, split, mm, n >> 6, n & 63, v[0], v[1]);
+    __syncthreads();
+    if (!s_last) return;
+    for (int r = tid >> 4; r < M * U; r += kGmThreads / 16) {
+      const int mm = r / U, b = r - mm * U, n = (it0 * U + b) * 16 + l16;
+      float v[2] = {0.0f, 0.0f};
+      for (int s0 = 0; s0 < p.nks; s0 += 8) {   // 8 slices in flight; past the last: the last again, not added
+        float t[8][GEGLU ? 2 : 1];
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+#pragma unroll
+          for (int h = 0; h < (GEGLU ? 2 : 1); ++h) t[u][h] = ldf<true>(slice_at(min(s0 + u, p.nks - 1), mm, b, h));
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+          if (s0 + u < p.nks)
+#pragma unroll
+            for (int h = 0; h < (GEGLU ? 2 : 1); ++h) v[h] += t[u][h];
+      }
+      epilogue<false>(p, split, mm, n >> 6, n & 63, v[0], v[1]);
+    }
   }
 }
 
 // Splits of several passes: a slice of whole passes per workgroup, as many slices as leave every workgroup one item and a CU
 // of its own
-static void slice_plan(const GemvP& p, GmPlan& pl) {
-  GmP& g = pl.args;
+static GmSliceP slice_plan(const GemvP& p, const GmPlan& pl) {
+  GmSliceP g{};
+  (GmP&)g = pl.args;
   const int passes = (min(p.kPer, p.K) + kGmPass - 1) / kGmPass, wgs = g.items * p.nsplit;
-  const int most = wgs <= 256 ? 256 / wgs : 1;
+  const int most = wgs <= 256 ? 256 / wgs : 1;   // gm_plan gives a workgroup more items than one only past 256
   g.pps = (passes + most - 1) / most;
   g.nks = (passes + g.pps - 1) / g.pps;
   g.part = ctx().part;      // at most 256 workgroups' 16 x 64 sums (a geglu's 16 x 32 twice): 1 MiB of its 64
   g.cnt = ctx().counters;   // nsplit * items <= 256
-  pl.grid.y = (unsigned)(p.nsplit * g.nks);   // gm_plan gives a workgroup more items than one only past 256
+  return g;
 }
 
+template <int ENC, bool SLICED>
+static void launch_form(const GemvP& p, const GmPlan& pl, dim3 grid, const typename GmArgs<SLICED>::type& g, hipStream_t s) {
+  const bool geglu = p.epi == P0_EPI_GEGLU, pleg = p.pro == P0_PRO_PLEG;
+#define P0_GM(NBK, GEGLU) (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true, SLICED> : gemvm_kernel<ENC, NBK, GEGLU, false, SLICED>)
+  auto k = geglu ? (pl.nbk == 4 ? P0_GM(4, true) : P0_GM(2, true))
+                 : pl.nbk == 4 ? P0_GM(4, false) : pl.nbk == 2 ? P0_GM(2, false) : P0_GM(1, false);
+#undef P0_GM
+  hipLaunchKernelGGL(k, grid, dim3(kGmThreads), 0, s, g);
+}
 template <int ENC>
 static void launch_enc(const GemvP& p, hipStream_t s) {
-  GmPlan pl = gm_plan(p, 512);
-  GmP& g = pl.args;
-  slice_plan(p, pl);
-  const bool geglu = p.epi == P0_EPI_GEGLU;
-  const int nbk = pl.nbk;
-  const bool pleg = p.pro == P0_PRO_PLEG, sliced = g.nks > 1;
-#define P0_GM(NBK, GEGLU)                                                                                               \
-  (sliced ? (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true, true> : gemvm_kernel<ENC, NBK, GEGLU, false, true>)             \
-          : (pleg ? gemvm_kernel<ENC, NBK, GEGLU, true, false> : gemvm_kernel<ENC, NBK, GEGLU, false, false>))
-  auto k = geglu ? (nbk == 4 ? P0_GM(4, true) : P0_GM(2, true))
-                 : nbk == 4 ? P0_GM(4, false) : nbk == 2 ? P0_GM(2, false) : P0_GM(1, false);
-#undef P0_GM
-  hipLaunchKernelGGL(k, pl.grid, dim3(kGmThreads), 0, s, g);
+  const GmPlan pl = gm_plan(p, 512);
+  const GmSliceP g = slice_plan(p, pl);
+  if (g.nks > 1) launch_form<ENC, true>(p, pl, dim3(pl.grid.x, pl.grid.y * g.nks), g, s);
+  else launch_form<ENC, false>(p, pl, pl.grid, pl.args, s);
 }
 
 // q4 calls of few rows that gemv.hip's fp32 kernel (x' staged once a workgroup, K over workgroups) runs faster. The line was

@@ -17,8 +17,6 @@ struct GmP {
   int N, K, kPer, M, pro, nsrc, items, ipw, wgs;   // wgs: workgroups per split
   int epi, NT; float cap;
   float* Y; float* MX; int64_t ldy, ldm;
-  int nks, pps;                      // gemvm.hip: K slices per split, over workgroups, and the passes of a slice
-  float* part; unsigned* cnt;        // nks > 1: the slices' sums and the arrival counts (the split-K workspace)
 };
 
 struct GmPlan {
