@@ -213,14 +213,18 @@ int p0_q4_dequant(const void* w, int64_t w_off, int64_t N, int64_t K, float* out
 /* knob 0: waves a GEMV call aims for before it splits K (default 2048);
  * knob 1: output tiles from which a GEMV wave streams two tiles (default 1024);
  * knob 2: fewest q4 groups a wave streams when K is split (default 2);
- * knob 3: most waves sharing one tile slot's K range inside a workgroup (default 16, at most 16; 8 when M > 2);
- * knob 4: fewest x rows M from which a gemvM call outside a chain runs on the matrix cores (default 2, i.e. every M > 1;
- *         17: never, both encodings on the fp32 VALU kernels). The matrix cores take x' as a pair of fp16 values under a
- *         power-of-two scale per row: 22 bits of every x' within 2^-18 of the row's largest, fewer below, where the VALU
- *         kernels take all 24. Knobs 0-3 plan the q4 VALU kernel; the matrix-core kernel and most calls at M = 1 split K
- *         over the waves of a workgroup only.
- * knob 5: K-slices per split of a q8g64s.t64 gemv (M = 1, splits of 2112-3072 k) across workgroups (default 0: planned,
- *         up to ~192 workgroups with at least 8 groups of 64 k a slice; a negative value restores the plan).
+ * knob 3: most waves sharing one tile slot's K range inside a workgroup (default 16, at most 16; 8 when M > 1);
+ * knob 4: fewest x rows M from which a gemvM call outside a chain may run on the matrix cores (default 2; 17: never, both
+ *         encodings on the fp32 VALU kernels). From there on q8 calls and q4 calls of more than 5 rows all do; q4 calls
+ *         of 2-5 rows but for those that the VALU kernel runs faster (short splits of many rows, long splits of many
+ *         blocks). The matrix cores take x' as a pair of fp16 values under a power-of-two scale per row: 22 bits of
+ *         every x' within 2^-18 of the row's largest, fewer below, where the VALU kernels take all 24. Knobs 0-3 plan
+ *         the q4 VALU kernel; the matrix-core kernel cuts K over workgroups only in whole passes of 2048 k, and most
+ *         calls at M = 1 split it over the waves of a workgroup only.
+ * knob 5: K-slices per split of a q8g64s.t64 gemv across workgroups, where the 16-wave kernel runs it: M = 1, splits of
+ *         2112-3072 k, and of 1024-2048 k a softcap of 1024 k or of at most 1024 rows and a geglu of 1024 k and more
+ *         than 4096 outputs. Default 0: planned, up to ~192 workgroups with at least 8 groups of 64 k a slice; a
+ *         negative value restores the plan.
  * value <= 0 only queries (knob 5: value < 0 restores its plan). Returns the previous value, or -1 for an unknown
  * knob. */
 int p0_gemv_tune(int knob, int value);

@@ -9,7 +9,7 @@
 // a quarter of one (q8), so it needs the group's 32 x' (its quarter's 16): the wave loads its 256 x' once (4 a lane),
 // applies the prologue, and hands them round through 1 KB of LDS into registers that serve every block.
 // Bound: the memory round trips of one launch (arguments, x, records, the stores), about 2.8 us between launches of a
-// recording; for the large ops, HBM. Per launch, recorded over weights in HBM (before: gemv.hip's kernel with its 500
+// recording; for the large ops, HBM. Per launch, recorded over a ring of weights (before: gemv.hip's kernel with its 500
 // bytes of arguments read in four serial steps, x' staged by every workgroup element by element, K sliced over workgroups
 // with partials in uncached memory; q8: gemv_q8.hip's): q4 gate_up 2 x 8192 x 2048 9.6 -> 6.9 us, 3072 x 2048 6.2 -> 3.3,
 // 2048 x 2048 5.8 -> 3.2, 2048 x 8192 in 4 splits 7.0 -> 4.9, 256 x 2048 5.2 -> 2.8, 65536 x 2048 20.8 -> 18.9; q8 5120 x

@@ -264,8 +264,8 @@ struct Rec {
   uint32_t sm;
 };
 
-// ---- the matrix-core arithmetic of chains with M > 1 rows (and, with a scale per row, of gemvm.hip). Per q4 group and 16 weight rows, two v_mfma_f32_16x16x32_f16
-// compute D[m][n] = 2^8 sum_k x'[m][k] q[n][k]: the A operand holds 2^8 x' split into fp16 hi + lo (2^8 x' = hi + lo to
+// ---- the matrix-core arithmetic of the pipelined chains with M > 1 rows (gemvm.hip has the same operands under a scale
+// per row). Per q4 group and 16 weight rows, two v_mfma_f32_16x16x32_f16 compute D[m][n] = 2^8 sum_k x'[m][k] q[n][k]: the A operand holds 2^8 x' split into fp16 hi + lo (2^8 x' = hi + lo to
 // 2^-22), the B operand the codes as exact fp16 values q (even k) and 16 q (odd k, whose x' carry the 1/16). Every
 // operand is a normal fp16 number: the codes come out of a code word as 1024 + q (the masked nibbles with the exponent
 // of 1024 OR-ed in, one v_and_or_b32 per pair) minus 1024, and the 2^8 keeps lo normal down to |x'| ~ 2^-11. (Fed as
@@ -273,7 +273,7 @@ struct Rec {
 // ~3e-7 to 3.4e-6 relative L2 off the M = 1 row on MI355X: the matrix cores do not take fp16 subnormals at full
 // precision.)
 // Rounding: these rows are not bit-identical to the fp32 VALU path's (which p0_q4_gemv and the chain kernels use);
-// they agree to ~3e-7 relative L2. Standalone launches stay on the VALU with p0_gemv_tune knob 4 = 17.
+// they agree to ~3e-7 relative L2.
 // Lane l holds D[4 (l / 16) + i][l % 16]: one weight row per lane, so each lane applies its row's scale and min
 // (2^-8 s D + m sum x') in fp32.
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
@@ -949,9 +949,9 @@ chain_kernel_t pick_chain_m(int W) {   // 16-wave chain workgroups for M = 1, 8-
   return q4_gemv_chain_kernel<M, 8>;
 }
 
-// the q8g64s.t64 GEMV (M = 1, gemv_q8.hip): the kernels and their LDS bytes
+// the q8g64s.t64 GEMV off the matrix cores (gemv_q8.hip): the kernels and their LDS bytes
 typedef void (*q8_kernel_t)(GemvP);
-q8_kernel_t q8_kernel();
+q8_kernel_t q8_kernel();            // an x row per grid.z
 q8_kernel_t q8_gemv1(bool geglu);   // M = 1, splits of at most 3072 k: 16 waves, the records in flight together
 size_t q8_gemv1_lds_bytes();
 size_t q8_lds_bytes();

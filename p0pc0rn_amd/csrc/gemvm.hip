@@ -23,11 +23,13 @@
 //    11.3 -> 7.0 us, 512 x 16384 17.0 -> 8.6, geglu 512 x 8192 17.9 -> 9.9 (before: the kernel that cut K over
 //    workgroups for every call; without slices 14.5, 27.2 and 22.5).
 // Bound: at the E2B shapes, one launch's chain (arguments, x, the split of x', the records, the reduction, the stores);
-// for a head, HBM. Per launch, recorded over weights in HBM, 5 rows: q4 gate_up 2 x 8192 x 2048 11.1 us (18.4 before: x'
+// for a head, HBM. Per launch, recorded over a ring of weights, 5 rows: q4 gate_up 2 x 8192 x 2048 11.1 us (18.4 before: x'
 // staged in LDS by every workgroup, K split over two workgroups with partials in uncached memory), 3072 x 2048 6.7 (11.0),
 // 2048 x 8192 in 4 splits 7.4 (13.4), 262144 x 2048 86 us = 3.9 TB/s (95); 16 rows: gate_up 12.2 (38.4). q8, where 4 waves a
 // tile took one group after another on the VALU: 5120 x 1536 7.2 (52.4), geglu 6144 x 1536 10.0 (91.5), 16 rows 11.7
-// (184). Relative L2 against float64: 1.2e-7 (q8; 3.8e-7 before), 1.7e-7 (q4; 1.9e-7).
+// (184). A ring that the last-level cache holds and one far past it read nearly alike: gate_up 11.2 over 168 MB, 11.0 over
+// 672; q8 5120 x 1536 7.0 over 194 MB, 7.4 over 584. Relative L2 against float64: 1.2e-7 (q8; 3.8e-7 before), 1.7e-7 (q4;
+// 1.9e-7).
 // Tried: the min term as a product of its own on the matrix cores (half the fp32 FMAs): 5% faster for the head, 3% slower
 // for the small ops, and its fp16 split of the group sums raised the error to 2.2e-7.
 #include "gemvm.hpp"
@@ -49,7 +51,7 @@ __device__ __forceinline__ half8_t codes_q8(uint32_t w0, uint32_t w1) {
   return __builtin_bit_cast(half8_t, u);
 }
 
-// The arguments of a launch in K slices (on their own: 24 bytes more for every launch cost the others 1%)
+// The arguments of a launch in K slices (a kernel without slices reads GmP alone)
 struct GmSliceP : GmP {
   int nks, pps;                // K slices per split, over workgroups, and the passes of a slice
   float* part; unsigned* cnt;  // the slices' sums and the arrival counts (the split-K workspace)
